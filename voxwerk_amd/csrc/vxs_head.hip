@@ -1,30 +1,27 @@
 // vxs_head.hip — the logit heads on the GPU, the step before the sampler.
 //
-// CodecHead and CodePredictorHead (src/Voxwerk/Talker/TalkerModel.cs:133-137) multiply a few fp32
-// hidden rows by a bf16 weight (the checkpoint's [out, in] layout, WeightPrecision.BFloat16,
-// DecoderStack.cs:7-15): out[r][n] = sum_k x[r][k] * W[n][k]. With the rows of a decode step
-// (1-24) this is a GEMV; the logits stay in HBM for the sampler. From 8 rows the matrix cores take it
-// (head_mfma_kernel, with x split exactly into three bf16 parts); below, the VALU form with fp32
-// products.
+// CodecHead and CodePredictorHead (src/Voxwerk/Talker/TalkerModel.cs:133-137) multiply fp32 hidden
+// rows by a bf16 weight (the checkpoint's [out, in] layout, WeightPrecision.BFloat16,
+// DecoderStack.cs:7-15): out[r][n] = sum_k x[r][k] * W[n][k]; the logits stay in HBM for the sampler.
+// One to three rows are a GEMV on the VALU; from there the matrix cores take it (x split exactly into
+// three bf16 parts): a split-K form while the call has few tiles, a tiled form for large batches
+// (launch_head has the rule and what it was measured on).
 //
-// VALU layout: a wave owns R = 8 consecutive outputs (4 when k > 1024, 2 for one or two rows); lane l
-// holds W[n][k] for k = 512 j + 8 l + 0..7
+// VALU layout: a wave owns two consecutive outputs; lane l holds W[n][k] for k = 512 j + 8 l + 0..7
 // (one 16-byte load per output and j, 1 KiB contiguous per wave instruction), all of its rows in
 // registers for the whole call. Per hidden row the lane loads its x slice (the next row's loads
-// issued before the current row's products), forms 8 partial dots and reduces them across the
-// wave by halving exchanges (xor 32, 16, 8: each lane keeps half of its partials and adds its
-// partner's other half) and then plain butterflies (xor 4, 2, 1): with R = 8, lane l ends with
-// output 4 b5 + 2 b4 + b3 of the wave, summed over all 64 lanes. The fp32 sum order is this kernel's own;
-// it differs from the reference's AVX-512 order by rounding only (bounded by K 2^-24 sum |x w|).
+// issued before the current row's products), forms its partial dots and reduces them across the wave by
+// a halving exchange (xor 32: each lane keeps one of the two outputs and adds its partner's copy of it)
+// and then plain butterflies (xor 16 .. 1). The fp32 sum order is each kernel's own; it differs from the
+// reference's AVX-512 order by rounding only (bounded by K 2^-24 sum |x w|).
 //
 // The int8 form (WeightPrecision.Int8, DecoderStack.cs:7-16) keeps W as q[n][k] in [-127, 127] and
 // one fp32 scale per output (PackedMatrix.FromBf16LinearInt8, PackedMatrix.cs:124-154):
 // out[r][n] = scale[n] * sum_k x[r][k] * q[n][k], the scale applied to the fp32 dot as the decode
-// path does (Gemm.cs:650-680, PanelPairDotInt8 / PanelDotInt8). Same layout and reduction, half the
-// weight bytes; a lane widens its int8 slice to fp32 once (exact) and keeps it in registers for
-// every row, so a row costs one FMA per weight. The packing itself runs on the GPU too
-// (head_pack_i8_kernel): per output the largest |w|, scale = amax / 127 (1 for an all-zero row),
-// q = clamp(round-half-even(w * (1 / scale)), -127, 127), all in correctly rounded fp32.
+// path does (Gemm.cs:650-680, PanelPairDotInt8 / PanelDotInt8). Same layouts and reductions, half the
+// weight bytes. The packing itself runs on the GPU too (head_pack_i8_kernel): per output the largest
+// |w|, scale = amax / 127 (1 for an all-zero row), q = clamp(round-half-even(w * (1 / scale)), -127,
+// 127), all in correctly rounded fp32.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -80,49 +77,20 @@ __device__ __forceinline__ XSlice<KJ> load_x(const HeadArgs& h, int m, int lane)
     return r;
 }
 
-// One halving exchange over lane bit `mask`: of 2H partials (outputs 2H apart in the lane pair),
-// each lane keeps the half its bit selects and adds the partner's copy of it.
-template <int H>
-__device__ __forceinline__ void halve(const float (&in)[2 * H], float (&out)[H], int lane, int mask) {
-    const bool bit = (lane & mask) != 0;
+// The wave's two partial dots of one row, reduced: lanes 0..31 end with the first, 32..63 the second.
+__device__ __forceinline__ float reduce_outputs(const float (&v)[2], int lane) {
+    const bool hi = lane >= 32;
+    float sum = (hi ? v[1] : v[0]) + __shfl_xor(hi ? v[0] : v[1], 32);
 #pragma unroll
-    for (int i = 0; i < H; i++) {
-        const float lo = in[i], hi = in[i + H];
-        out[i] = (bit ? hi : lo) + __shfl_xor(bit ? lo : hi, mask);
-    }
-}
-
-// The wave's R partial dots of one row reduced to one output per lane group (see the layout note).
-template <int R>
-__device__ __forceinline__ float reduce_outputs(const float (&v)[R], int lane) {
-    constexpr int kGroup = 64 / R;
-    float sum;
-    if constexpr (R == 8) {
-        float q[4], t[2], s1[1];
-        halve<4>(v, q, lane, 32);
-        halve<2>(q, t, lane, 16);
-        halve<1>(t, s1, lane, 8);
-        sum = s1[0];
-    } else if constexpr (R == 4) {
-        float q[2], s1[1];
-        halve<2>(v, q, lane, 32);
-        halve<1>(q, s1, lane, 16);
-        sum = s1[0];
-    } else {
-        float s1[1];
-        halve<1>(v, s1, lane, 32);
-        sum = s1[0];
-    }
-#pragma unroll
-    for (int mask = kGroup / 2; mask >= 1; mask /= 2) sum += __shfl_xor(sum, mask);
+    for (int mask = 16; mask >= 1; mask /= 2) sum += __shfl_xor(sum, mask);
     return sum;
 }
 
-// R outputs per wave (8 or 4), KJ slices of 8 per lane (k <= 512 KJ).
-template <int KJ, int R, bool FULL>
+constexpr int R = 2;  // outputs per wave
+
+// KJ slices of 8 per lane (k <= 512 KJ).
+template <int KJ, bool FULL>
 __global__ __launch_bounds__(kHT) void head_kernel(HeadArgs a) {
-    static_assert(R == 8 || R == 4 || R == 2, "eight, four or two outputs per wave");
-    constexpr int kGroup = 64 / R;  // lanes that share an output after the halving exchanges
     const int lane = threadIdx.x & 63;
     const int n0 = (blockIdx.x * (kHT / 64) + (threadIdx.x >> 6)) * R;
     if (n0 >= a.n) return;  // whole wave past the last output (wave-uniform)
@@ -141,19 +109,10 @@ __global__ __launch_bounds__(kHT) void head_kernel(HeadArgs a) {
             w[o][j] = in ? v : u4{0u, 0u, 0u, 0u};
         }
 
-    // output this lane holds after the halving exchanges (lane bits 5, 4[, 3], most significant first)
-    const int o_mine = R == 8   ? 4 * ((lane >> 5) & 1) + 2 * ((lane >> 4) & 1) + ((lane >> 3) & 1)
-                       : R == 4 ? 2 * ((lane >> 5) & 1) + ((lane >> 4) & 1)
-                                : (lane >> 5) & 1;
+    const int o_mine = lane >> 5;  // the output this lane holds after the reduction
     // rows two at a time with two slice buffers, each reloaded in place while the other is used,
     // so a row's loads are in flight during the previous row's products and exchanges
     auto row = [&](int m, const XSlice<KJ>& x) {
-        if constexpr (KJ > 2) {  // keep the weights packed (widened per row): half the registers
-#pragma unroll
-            for (int o = 0; o < R; o++)
-#pragma unroll
-                for (int j = 0; j < KJ; j++) asm volatile("" : "+v"(w[o][j]));
-        }
         float v[R];
 #pragma unroll
         for (int o = 0; o < R; o++) {
@@ -162,8 +121,8 @@ __global__ __launch_bounds__(kHT) void head_kernel(HeadArgs a) {
             for (int j = 0; j < KJ; j++) acc = dot8(w[o][j], x.a[j], x.b[j], acc);
             v[o] = acc;
         }
-        const float sum = reduce_outputs<R>(v, lane);
-        if ((lane & (kGroup - 1)) == 0 && n0 + o_mine < a.n) a.out[(int64_t)m * a.ldo + n0 + o_mine] = sum;
+        const float sum = reduce_outputs(v, lane);
+        if ((lane & 31) == 0 && n0 + o_mine < a.n) a.out[(int64_t)m * a.ldo + n0 + o_mine] = sum;
     };
     // this workgroup's rows: group blockIdx.y of a.row_group rows
     const int first = blockIdx.y * a.row_group;
@@ -180,11 +139,9 @@ __global__ __launch_bounds__(kHT) void head_kernel(HeadArgs a) {
 
 typedef unsigned int u2 __attribute__((ext_vector_type(2)));
 
-// int8 weights, widened once: R outputs per wave, KJ slices of 8 per lane (k <= 512 KJ).
-template <int KJ, int R, bool FULL>
+// int8 weights, widened once: KJ slices of 8 per lane (k <= 512 KJ).
+template <int KJ, bool FULL>
 __global__ __launch_bounds__(kHT) void head_i8_kernel(HeadArgs a) {
-    static_assert(R == 8 || R == 4 || R == 2, "eight, four or two outputs per wave");
-    constexpr int kGroup = 64 / R;
     const int lane = threadIdx.x & 63;
     const int n0 = (blockIdx.x * (kHT / 64) + (threadIdx.x >> 6)) * R;
     if (n0 >= a.n) return;  // whole wave past the last output (wave-uniform)
@@ -217,9 +174,7 @@ __global__ __launch_bounds__(kHT) void head_i8_kernel(HeadArgs a) {
                 w[o][j][i] = in ? f : 0.0f;
             }
         }
-    const int o_mine = R == 8   ? 4 * ((lane >> 5) & 1) + 2 * ((lane >> 4) & 1) + ((lane >> 3) & 1)
-                       : R == 4 ? 2 * ((lane >> 5) & 1) + ((lane >> 4) & 1)
-                                : (lane >> 5) & 1;
+    const int o_mine = lane >> 5;
     const float sc = a.scale[min(n0 + o_mine, a.n - 1)];
     auto row = [&](int m, const XSlice<KJ>& x) {
         float v[R];
@@ -234,8 +189,8 @@ __global__ __launch_bounds__(kHT) void head_i8_kernel(HeadArgs a) {
             }
             v[o] = acc;
         }
-        const float sum = reduce_outputs<R>(v, lane) * sc;
-        if ((lane & (kGroup - 1)) == 0 && n0 + o_mine < a.n) a.out[(int64_t)m * a.ldo + n0 + o_mine] = sum;
+        const float sum = reduce_outputs(v, lane) * sc;
+        if ((lane & 31) == 0 && n0 + o_mine < a.n) a.out[(int64_t)m * a.ldo + n0 + o_mine] = sum;
     };
     const int first = blockIdx.y * a.row_group;
     const int last = min(a.rows, first + a.row_group) - 1;
@@ -249,7 +204,7 @@ __global__ __launch_bounds__(kHT) void head_i8_kernel(HeadArgs a) {
     }
 }
 
-// ---- matrix-core form, for 8 or more rows -------------------------------------------------------
+// ---- matrix-core forms, for 8 or more rows ------------------------------------------------------
 // The hidden rows are fp32 and v_mfma_f32_16x16x32_bf16 multiplies bf16, so each x is split exactly
 // into three bf16 parts, x = h + m + l: h keeps the top 8 significand bits (truncation), m the next
 // 8 of the remainder x - h (exact in fp32), l what is left (at most 8 bits: exact in bf16), exact
@@ -258,58 +213,40 @@ __global__ __launch_bounds__(kHT) void head_i8_kernel(HeadArgs a) {
 // of at most 3 K / 32 + 2 matrix operations and NW wave partials per output; the test bound is that
 // of K sequential fp32 additions). An int8 weight widens to bf16 exactly (|q| <= 127).
 //
-// Tile: a workgroup owns 16 TM outputs and all rows, 32 at a time; its NW waves split K in chunks
-// of 64 (two 32-deep steps), chunk c to wave c % NW, and their 16 TM x 32 partial sums are added in
-// LDS in wave order. MFMA operand layout (16x16x32): lane l supplies A[l % 16][8 (l / 16) + 0..7] and
+// +-inf and NaN need no care in the split: such an x (its remainders are NaN) or weight (inf times a
+// zero part is NaN) leaves NaN in its outputs, and an output that is not finite is formed again by
+// output_in_order, whose products and sums follow IEEE. Finite outputs had finite operands.
+//
+// MFMA operand layout (16x16x32): lane l supplies A[l % 16][8 (l / 16) + 0..7] and
 // B[8 (l / 16) + 0..7][l % 16], and holds C[4 (l / 16) + i][l % 16], i = 0..3. Here A = W (outputs by
-// k), B = x^T (k by rows), so lane l reads 8 consecutive k of one weight row and of one hidden row.
+// k), B = x^T (k by rows), so lane l reads 8 consecutive k of one weight row and of one hidden row and
+// ends with four consecutive outputs of one hidden row. Tile rows past the last hidden row or output
+// read the last one (each result depends on its own row of A and column of B alone; what they
+// compute is not stored); past the end of k the hidden values are zero.
 typedef __bf16 bf8 __attribute__((ext_vector_type(8)));
 
-// three exact bf16 parts of 8 fp32 values. With NONFINITE, +-inf and NaN are their own high part (a
-// NaN keeps a payload bit in the bf16 half) with zero remainders, so the products follow IEEE
-// (inf w = +-inf, inf 0 = NaN, NaN w = NaN); without it such a value would turn into NaN parts.
-template <bool NONFINITE>
-__device__ __forceinline__ void split3(const f4& a, const f4& b, bf8& h, bf8& m, bf8& l) {
+// three exact bf16 parts of 8 finite fp32 values
+struct Parts {
+    u4 h, m, l;
+};
+__device__ __forceinline__ Parts split3(const f4& a, const f4& b) {
     const float v[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
     uint32_t th[8], tm[8], tl[8];
 #pragma unroll
     for (int i = 0; i < 8; i++) {
-        const uint32_t u = __float_as_uint(v[i]);
-        float r1;
-        if constexpr (NONFINITE) {
-            const bool fin = (u & 0x7F800000u) != 0x7F800000u;
-            th[i] = fin || !(u & 0x007FFFFFu) ? u & 0xFFFF0000u : u | 0x00400000u;
-            r1 = fin ? v[i] - __uint_as_float(th[i]) : 0.0f;
-        } else {
-            th[i] = u & 0xFFFF0000u;
-            r1 = v[i] - __uint_as_float(th[i]);
-        }
-        tm[i] = __float_as_uint(r1) & 0xFFFF0000u;
-        tl[i] = __float_as_uint(r1 - __uint_as_float(tm[i]));
+        th[i] = __float_as_uint(v[i]);
+        const float r1 = v[i] - __uint_as_float(th[i] & 0xFFFF0000u);
+        tm[i] = __float_as_uint(r1);
+        tl[i] = __float_as_uint(r1 - __uint_as_float(tm[i] & 0xFFFF0000u));
     }
-    u4 ph, pm, pl;
+    Parts p;
 #pragma unroll
     for (int i = 0; i < 4; i++) {  // high halves of elements 2i (low) and 2i + 1 (high)
-        ph[i] = __builtin_amdgcn_perm(th[2 * i + 1], th[2 * i], 0x07060302u);
-        pm[i] = __builtin_amdgcn_perm(tm[2 * i + 1], tm[2 * i], 0x07060302u);
-        pl[i] = __builtin_amdgcn_perm(tl[2 * i + 1], tl[2 * i], 0x07060302u);
+        p.h[i] = __builtin_amdgcn_perm(th[2 * i + 1], th[2 * i], 0x07060302u);
+        p.m[i] = __builtin_amdgcn_perm(tm[2 * i + 1], tm[2 * i], 0x07060302u);
+        p.l[i] = __builtin_amdgcn_perm(tl[2 * i + 1], tl[2 * i], 0x07060302u);
     }
-    h = __builtin_bit_cast(bf8, ph);
-    m = __builtin_bit_cast(bf8, pm);
-    l = __builtin_bit_cast(bf8, pl);
-}
-
-// split3 with the non-finite handling only when the wave holds such a value (one class test per
-// value; the rare case takes the longer form)
-__device__ __forceinline__ void split3_any(const f4& a, const f4& b, bf8& h, bf8& m, bf8& l) {
-    bool nf = false;
-#pragma unroll
-    for (int i = 0; i < 4; i++)
-        nf |= __builtin_amdgcn_class(a[i], 0x207) | __builtin_amdgcn_class(b[i], 0x207);  // NaN, +-inf
-    if (__ballot(nf))
-        split3<true>(a, b, h, m, l);
-    else
-        split3<false>(a, b, h, m, l);
+    return p;
 }
 
 // 8 int8 weights (two dwords) as 8 bf16: the biased byte converted, 128 subtracted (exact), the
@@ -327,105 +264,391 @@ __device__ __forceinline__ bf8 i8_to_bf16(uint32_t lo, uint32_t hi) {
     return __builtin_bit_cast(bf8, p);
 }
 
-template <int TM, int NW, bool I8>
-__global__ __launch_bounds__(64 * NW) void head_mfma_kernel(HeadArgs a) {
-    __shared__ f4 part[NW][TM * 2][64];  // each wave's accumulators, per (output tile, row tile)
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+// Operands reach the matrix cores through LDS. A wave's 16 consecutive lanes want 16 different rows,
+// and loads in that order cost a cache line per lane (measured per compute unit, rows of 2 KiB that
+// hit the L2: 16 rows x 64 bytes per wave load 27 bytes per ns, 8 rows x 128 bytes 78). So a tile of 16
+// rows x 64 k is loaded with consecutive lanes along k (whole lines), written to LDS and read back one
+// fragment per lane; the 16-byte units of a row are placed at their index xor the row, so eight
+// consecutive lanes touch all 32 banks once in either order.
+//
+// Loads are raw buffer loads from the first row of the workgroup's tile: entries past the last row, or
+// past k (an offset out of range), read as zero without touching memory. Offsets are 32-bit, which
+// mfma_fits checks.
+template <bool I8>
+using WRaw = typename std::conditional<I8, u2, u4>::type;  // 8 weights as loaded
+constexpr uint32_t kOut = 0x80000000u;                       // an offset past every tile
+
+struct Tile {
+    __amdgpu_buffer_rsrc_t rsrc;
+    uint32_t ld;  // row length in bytes
+};
+__device__ __forceinline__ Tile tile_of(const void* base, int64_t ld_bytes, int row0, int rows, int row_bytes) {
+    const uint32_t ld = (uint32_t)ld_bytes;
+    const char* p = static_cast<const char*>(base) + (int64_t)row0 * ld_bytes;
+    return {__builtin_amdgcn_make_buffer_rsrc((void*)p, (short)0, (int)((uint32_t)(rows - 1) * ld + (uint32_t)row_bytes), 0x00020000),
+            ld};
+}
+// the 8 weights of tile row `row` from k on (k >= K: zeros)
+template <bool I8>
+__device__ __forceinline__ WRaw<I8> load_w8(const Tile& t, uint32_t row_off, int k, int K) {
+    const uint32_t off = k < K ? row_off + (uint32_t)k * (I8 ? 1u : 2u) : kOut;
+    if constexpr (I8)
+        return __builtin_bit_cast(u2, __builtin_amdgcn_raw_buffer_load_b64(t.rsrc, off, 0, 0));
+    else
+        return __builtin_bit_cast(u4, __builtin_amdgcn_raw_buffer_load_b128(t.rsrc, off, 0, 0));
+}
+__device__ __forceinline__ f4 load_x4(const Tile& t, uint32_t row_off, int k, int K) {
+    const uint32_t off = k < K ? row_off + 4u * (uint32_t)k : kOut;
+    return __builtin_bit_cast(f4, __builtin_amdgcn_raw_buffer_load_b128(t.rsrc, off, 0, 0));
+}
+// Keeps the compiler from reordering a wave's LDS accesses. The hardware executes them in order, so a
+// buffer of the wave's own is written again as soon as its reads are issued, with no wait.
+__device__ __forceinline__ void wave_order() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+template <bool I8>
+__device__ __forceinline__ bf8 w_operand(const WRaw<I8>& r) {
+    if constexpr (I8)
+        return i8_to_bf16(r.x, r.y);
+    else
+        return __builtin_bit_cast(bf8, r);
+}
+
+// One output in k order by fp32 FMAs, the int8 scale last: for results that are not finite.
+template <bool I8>
+__device__ __forceinline__ float output_in_order(const HeadArgs& a, int r, int n) {
+    const float* x = a.x + (int64_t)r * a.ldx;
+    float acc = 0.0f;
+#pragma unroll 1
+    for (int k = 0; k < a.k; k++) {
+        float w;
+        if constexpr (I8)
+            w = (float)(int)a.q[(int64_t)n * a.ldw + k];
+        else
+            w = __uint_as_float((uint32_t)a.w[(int64_t)n * a.ldw + k] << 16);
+        acc = __builtin_fmaf(w, x[k], acc);
+    }
+    if constexpr (I8) acc *= a.scale[n];
+    return acc;
+}
+__device__ __forceinline__ bool finite(float v) { return __builtin_fabsf(v) < __builtin_huge_valf(); }
+
+// XCD-aware tile order: workgroups go to the 8 XCDs in turn, each with an L2 of its own, so workgroup
+// b takes tile (b % 8) * per + b / 8 of the column-major tile list (row tiles fastest): an XCD's
+// workgroups then share a few column tiles of W, read from memory once per XCD. False past the end.
+__device__ __forceinline__ bool xcd_tile(int row_tiles, int tiles, int& rt, int& ct) {
+    const int per = (tiles + 7) / 8;
+    const int t = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
+    if ((int)(blockIdx.x >> 3) >= per || t >= tiles) return false;
+    rt = t % row_tiles;
+    ct = t / row_tiles;
+    return true;
+}
+inline int xcd_grid(int tiles) { return (tiles + 7) / 8 * 8; }
+
+// Split-K form, for calls with few tiles: a workgroup owns 16 CT outputs of 16 RT rows; its NW waves
+// split K in chunks of 64 (two 32-deep steps), chunk c to wave c % NW, each through operand buffers of
+// its own (no barrier before the end). A tile's registers take the next chunk's loads as soon as the
+// tile is in LDS. The waves' partial sums are added in LDS in a fixed order (waves w and w + NW / 2
+// first, then over w).
+template <int RT, int CT, int NW, bool I8>
+__global__ __launch_bounds__(64 * NW) void head_mfma_kernel(HeadArgs a, int row_tiles, int tiles) {
+    constexpr int NH = NW / 2;
+    struct Turn {
+        f4 x[16][16];
+        WRaw<I8> w[CT > 1 ? 2 : 1][16][8];
+    };
+    __shared__ union {
+        Turn turn[NW];
+        f4 part[NH][RT * CT][64];
+    } sm;
+    int rt, ct;
+    if (!xcd_tile(row_tiles, tiles, rt, ct)) return;
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int g = lane >> 4, c16 = lane & 15;
-    const int n0 = blockIdx.x * 16 * TM;
-    const int nchunks = (a.k + 63) / 64;
-    for (int r0 = 0; r0 < a.rows; r0 += 32) {
-        f4 acc[TM][2];
+    const int n0 = ct * 16 * CT, r0 = rt * 16 * RT;
+    const int K = a.k, nchunks = (K + 63) / 64;
+    const Tile tw = I8 ? tile_of(a.q, a.ldw, n0, min(16 * CT, a.n - n0), K)
+                       : tile_of(a.w, a.ldw * 2, n0, min(16 * CT, a.n - n0), 2 * K);
+    const Tile tx = tile_of(a.x, a.ldx * 4, r0, min(16 * RT, a.rows - r0), 4 * K);
+    // a wave load holds 8 weight rows x 8 k, or 4 hidden rows x 4 k, per lane
+    const uint32_t wl = (uint32_t)(lane >> 3) * tw.ld, xl = (uint32_t)(lane >> 4) * tx.ld;
+    const int kw = 8 * (lane & 7), kx = 4 * (lane & 15);
+    f4 acc[CT][RT];
 #pragma unroll
-        for (int tm = 0; tm < TM; tm++)
+    for (int t = 0; t < CT; t++)
 #pragma unroll
-            for (int tn = 0; tn < 2; tn++) acc[tm][tn] = f4{0.f, 0.f, 0.f, 0.f};
-        for (int c = wv; c < nchunks; c += NW) {
-            // every load of the chunk is issued before the first product: the weights of both steps
-            // and output tiles, the hidden rows' slices of both steps and row tiles (lane l: 8
-            // consecutive k from 64 c + 32 step + 8 (l / 16), weight row / hidden row l % 16 of the tile)
-            typedef typename std::conditional<I8, u2, u4>::type WRaw;
-            WRaw wr[2][TM];
-            f4 xr[2][2][2];
-            bool kin[2];
+        for (int q = 0; q < RT; q++) acc[t][q] = f4{0.f, 0.f, 0.f, 0.f};
+    WRaw<I8> wr[CT][2];
+    f4 xr[RT][4];
+    auto load_wt = [&](int c, int t) {
 #pragma unroll
-            for (int st = 0; st < 2; st++) {
-                const int k = 64 * c + 32 * st + 8 * g;  // k % 8 == 0: the 8 are all inside or all past k
-                kin[st] = k < a.k;
+        for (int j = 0; j < 2; j++) wr[t][j] = load_w8<I8>(tw, wl + (uint32_t)(16 * t + 8 * j) * tw.ld, 64 * c + kw, K);
+    };
+    auto load_xt = [&](int c, int q) {
 #pragma unroll
-                for (int tm = 0; tm < TM; tm++) {
-                    const int n = n0 + 16 * tm + c16;
-                    const int64_t off = (int64_t)min(n, a.n - 1) * a.ldw + (kin[st] ? k : 0);
-                    if constexpr (I8)
-                        wr[st][tm] = *reinterpret_cast<const u2*>(a.q + off);
-                    else
-                        wr[st][tm] = __builtin_nontemporal_load(reinterpret_cast<const u4*>(a.w + off));
-                }
+        for (int j = 0; j < 4; j++) xr[q][j] = load_x4(tx, xl + (uint32_t)(16 * q + 4 * j) * tx.ld, 64 * c + kx, K);
+    };
+    Turn& tb = sm.turn[wv];
+    if (wv < nchunks) {
 #pragma unroll
-                for (int tn = 0; tn < 2; tn++) {
-                    const int r = r0 + 16 * tn + c16;
-                    const float* px = a.x + (int64_t)min(r, a.rows - 1) * a.ldx + (kin[st] ? k : 0);
-                    xr[st][tn][0] = *reinterpret_cast<const f4*>(px);
-                    xr[st][tn][1] = *reinterpret_cast<const f4*>(px + 4);
-                }
+        for (int q = 0; q < RT; q++) load_xt(wv, q);
+#pragma unroll
+        for (int t = 0; t < CT; t++) load_wt(wv, t);
+    }
+#pragma unroll 1
+    for (int c = wv; c < nchunks; c += NW) {
+        const int nx = c + NW;  // past the last chunk its loads are out of range
+        Parts p[RT][2];
+#pragma unroll
+        for (int q = 0; q < RT; q++) {
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const int row = 4 * j + (lane >> 4);
+                tb.x[row][(lane & 15) ^ (row & 7)] = xr[q][j];
             }
+            wave_order();
+            f4 f[2][2];
 #pragma unroll
-            for (int st = 0; st < 2; st++) {
-                bf8 wa[TM];
+            for (int st = 0; st < 2; st++)
 #pragma unroll
-                for (int tm = 0; tm < TM; tm++) {
-                    const bool in = kin[st] && n0 + 16 * tm + c16 < a.n;
-                    if constexpr (I8)
-                        wa[tm] = i8_to_bf16(in ? wr[st][tm].x : 0u, in ? wr[st][tm].y : 0u);
-                    else
-                        wa[tm] = __builtin_bit_cast(bf8, in ? wr[st][tm] : u4{0u, 0u, 0u, 0u});
-                }
+                for (int h = 0; h < 2; h++) f[st][h] = tb.x[c16][(8 * st + 2 * g + h) ^ (c16 & 7)];
+            wave_order();
+            load_xt(nx, q);
 #pragma unroll
-                for (int tn = 0; tn < 2; tn++) {
-                    const bool in = kin[st] && r0 + 16 * tn + c16 < a.rows;
-                    const f4 z = {0.f, 0.f, 0.f, 0.f};
-                    bf8 h, m, l;
-                    split3_any(in ? xr[st][tn][0] : z, in ? xr[st][tn][1] : z, h, m, l);
-#pragma unroll
-                    for (int tm = 0; tm < TM; tm++) {
-                        acc[tm][tn] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wa[tm], h, acc[tm][tn], 0, 0, 0);
-                        acc[tm][tn] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wa[tm], m, acc[tm][tn], 0, 0, 0);
-                        acc[tm][tn] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wa[tm], l, acc[tm][tn], 0, 0, 0);
-                    }
-                }
-            }
+            for (int st = 0; st < 2; st++) p[q][st] = split3(f[st][0], f[st][1]);
         }
+        WRaw<I8> f[2][2];
+        auto turn_w = [&](int t) {
 #pragma unroll
-        for (int tm = 0; tm < TM; tm++)
-#pragma unroll
-            for (int tn = 0; tn < 2; tn++) part[wv][2 * tm + tn][lane] = acc[tm][tn];
-        __syncthreads();
-        // (output, row) pairs of the tile, consecutive threads on consecutive outputs: the waves'
-        // partials added in wave order, scaled (int8), stored
-        for (int p = threadIdx.x; p < 16 * TM * 32; p += 64 * NW) {
-            const int nl = p % (16 * TM), rl = p / (16 * TM);
-            const int tm = nl / 16, mi = nl % 16, tn = rl / 16;
-            const int l = 16 * (mi / 4) + rl % 16;
-            float sum = 0.f;
-#pragma unroll
-            for (int w = 0; w < NW; w++) sum += part[w][2 * tm + tn][l][mi % 4];
-            const int n = n0 + nl, r = r0 + rl;
-            if (n < a.n && r < a.rows) {
-                if constexpr (I8) sum *= a.scale[n];
-                a.out[(int64_t)r * a.ldo + n] = sum;
+            for (int j = 0; j < 2; j++) {
+                const int row = 8 * j + (lane >> 3);
+                tb.w[t & 1][row][(lane & 7) ^ (row & 7)] = wr[t][j];
             }
+            wave_order();
+#pragma unroll
+            for (int st = 0; st < 2; st++) f[t & 1][st] = tb.w[t & 1][c16][(4 * st + g) ^ (c16 & 7)];
+            wave_order();
+            load_wt(nx, t);
+        };
+        turn_w(0);
+#pragma unroll
+        for (int t = 0; t < CT; t++) {
+            if (t + 1 < CT) turn_w(t + 1);
+            bf8 wa[2];
+#pragma unroll
+            for (int st = 0; st < 2; st++) wa[st] = w_operand<I8>(f[t & 1][st]);
+            // the chunk's sums from zero, smallest parts first, then added to the wave's: six roundings of
+            // which three are of the size of the sum
+            f4 s[RT];
+#pragma unroll
+            for (int q = 0; q < RT; q++) s[q] = f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int part = 0; part < 3; part++)
+#pragma unroll
+                for (int st = 0; st < 2; st++)
+#pragma unroll
+                    for (int q = 0; q < RT; q++)
+                        s[q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                            wa[st], __builtin_bit_cast(bf8, part == 0 ? p[q][st].l : part == 1 ? p[q][st].m : p[q][st].h), s[q], 0, 0, 0);
+#pragma unroll
+            for (int q = 0; q < RT; q++) acc[t][q] += s[q];
         }
-        __syncthreads();  // the partials are read before the next row group writes them
+    }
+    __syncthreads();  // every wave is done with its operand buffers
+    if (wv >= NH)
+#pragma unroll
+        for (int t = 0; t < CT; t++)
+#pragma unroll
+            for (int q = 0; q < RT; q++) sm.part[wv - NH][t * RT + q][lane] = acc[t][q];
+    __syncthreads();
+    if (wv < NH)
+#pragma unroll
+        for (int t = 0; t < CT; t++)
+#pragma unroll
+            for (int q = 0; q < RT; q++) sm.part[wv][t * RT + q][lane] = acc[t][q] + sm.part[wv][t * RT + q][lane];
+    __syncthreads();
+    // (output, row) pairs of the tile, consecutive threads on consecutive outputs
+    for (int e = threadIdx.x; e < 16 * CT * 16 * RT; e += 64 * NW) {
+        const int nl = e % (16 * CT), rl = e / (16 * CT);
+        const int l = 16 * ((nl % 16) / 4) + rl % 16;
+        double dsum = 0.0;
+#pragma unroll
+        for (int w = 0; w < NH; w++) dsum += (double)sm.part[w][(nl / 16) * RT + rl / 16][l][nl % 4];
+        float sum = (float)dsum;
+        const int n = n0 + nl, r = r0 + rl;
+        if (n >= a.n || r >= a.rows) continue;
+        if constexpr (I8) sum *= a.scale[n];
+        if (!finite(sum)) sum = output_in_order<I8>(a, r, n);
+        a.out[(int64_t)r * a.ldo + n] = sum;
     }
 }
 
-template <int TM, int NW>
+template <int RT, int CT, int NW>
 hipError_t launch_mfma(const HeadArgs& a, hipStream_t stream) {
-    const dim3 grid((a.n + 16 * TM - 1) / (16 * TM));
+    const int row_tiles = (a.rows + 16 * RT - 1) / (16 * RT);
+    const int tiles = row_tiles * ((a.n + 16 * CT - 1) / (16 * CT));
     if (a.q)
-        hipLaunchKernelGGL((head_mfma_kernel<TM, NW, true>), grid, dim3(64 * NW), 0, stream, a);
+        hipLaunchKernelGGL((head_mfma_kernel<RT, CT, NW, true>), dim3(xcd_grid(tiles)), dim3(64 * NW), 0, stream, a, row_tiles, tiles);
     else
-        hipLaunchKernelGGL((head_mfma_kernel<TM, NW, false>), grid, dim3(64 * NW), 0, stream, a);
+        hipLaunchKernelGGL((head_mfma_kernel<RT, CT, NW, false>), dim3(xcd_grid(tiles)), dim3(64 * NW), 0, stream, a, row_tiles, tiles);
+    return hipGetLastError();
+}
+
+// Tiled form, for calls with tiles enough to fill the chip: a workgroup of 2 x 2 waves owns 32 WR rows
+// x 32 WC outputs, a wave 16 WR x 16 WC, over the whole of K in steps of 64. Both operands are staged
+// in LDS once per workgroup, the hidden rows split there into their three parts (int8 weights widened);
+// the next step's loads are in flight during a step's products, and other workgroups of the compute
+// unit fill the rest.
+template <int WR, int WC, bool I8>
+__global__ __launch_bounds__(kHT) __attribute__((amdgpu_waves_per_eu(2))) void head_mfma_tiled_kernel(HeadArgs a, int row_tiles,
+                                                                                                      int tiles) {
+    constexpr int BM = 32 * WR, BN = 32 * WC;
+    __shared__ u4 xs[3][BM][8], ws[BN][8];  // rows of 64 bf16, the 16-byte units of a row xor-ed with it
+    int rt, ct;
+    if (!xcd_tile(row_tiles, tiles, rt, ct)) return;
+    const int t = threadIdx.x, lane = t & 63, wv = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int g = lane >> 4, c16 = lane & 15;
+    const int r0 = rt * BM, n0 = ct * BN;
+    const int rw = (wv & 1) * 16 * WR, nw = (wv >> 1) * 16 * WC;  // the wave's part of the tile
+    const int K = a.k, nchunks = (K + 63) / 64;
+    const Tile tw = I8 ? tile_of(a.q, a.ldw, n0, min(BN, a.n - n0), K) : tile_of(a.w, a.ldw * 2, n0, min(BN, a.n - n0), 2 * K);
+    const Tile tx = tile_of(a.x, a.ldx * 4, r0, min(BM, a.rows - r0), 4 * K);
+    // a load of the workgroup holds 32 weight rows x 8 k, or 16 hidden rows x 4 k, per thread
+    const uint32_t wl = (uint32_t)(t >> 3) * tw.ld, xl = (uint32_t)(t >> 4) * tx.ld;
+    const int kw = 8 * (t & 7), kx = 4 * (t & 15);
+    // The sums of the high parts in acc, moved to tot every 128 k; those of the others, 2^-8 of their
+    // size, in low, which also takes what the addition to tot rounds off (Fast2Sum): so the roundings
+    // of the size of the sum are the four of each 128 k and the last. Relative 2-norm error against
+    // 64 bits, normal data, k = 1024: 0.7e-7 (the VALU form: 1.0e-7; one chain over all of k: 3.4e-7).
+    f4 acc[WC][WR], low[WC][WR], tot[WC][WR];
+#pragma unroll
+    for (int i = 0; i < WC; i++)
+#pragma unroll
+        for (int q = 0; q < WR; q++) acc[i][q] = low[i][q] = tot[i][q] = f4{0.f, 0.f, 0.f, 0.f};
+    WRaw<I8> wr[WC];
+    f4 xr[2 * WR];
+    auto load = [&](int c) {  // past the last chunk: out of range
+#pragma unroll
+        for (int j = 0; j < 2 * WR; j++) xr[j] = load_x4(tx, xl + (uint32_t)(16 * j) * tx.ld, 64 * c + kx, K);
+#pragma unroll
+        for (int j = 0; j < WC; j++) wr[j] = load_w8<I8>(tw, wl + (uint32_t)(32 * j) * tw.ld, 64 * c + kw, K);
+    };
+    load(0);
+#pragma unroll 1
+    for (int c = 0; c < nchunks; c++) {
+#pragma unroll
+        for (int j = 0; j < 2 * WR; j++) {
+            const int row = 16 * j + (t >> 4);
+            uint32_t th[4], tm[4], tl[4];
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                th[i] = __float_as_uint(xr[j][i]);
+                const float r1 = xr[j][i] - __uint_as_float(th[i] & 0xFFFF0000u);
+                tm[i] = __float_as_uint(r1);
+                tl[i] = __float_as_uint(r1 - __uint_as_float(tm[i] & 0xFFFF0000u));
+            }
+            const int unit = ((t & 15) >> 1) ^ (row & 7), half = t & 1;
+            auto put = [&](int part, const uint32_t (&v)[4]) {
+                reinterpret_cast<u2*>(&xs[part][row][unit])[half] = u2{__builtin_amdgcn_perm(v[1], v[0], 0x07060302u),
+                                                                       __builtin_amdgcn_perm(v[3], v[2], 0x07060302u)};
+            };
+            put(0, th);
+            put(1, tm);
+            put(2, tl);
+        }
+#pragma unroll
+        for (int j = 0; j < WC; j++) {
+            const int row = 32 * j + (t >> 3);
+            ws[row][(t & 7) ^ (row & 7)] = __builtin_bit_cast(u4, w_operand<I8>(wr[j]));
+        }
+        __syncthreads();
+        load(c + 1);
+#pragma unroll
+        for (int st = 0; st < 2; st++) {
+            const int unit = (4 * st + g) ^ (c16 & 7);
+            bf8 wa[WC];
+#pragma unroll
+            for (int i = 0; i < WC; i++) wa[i] = __builtin_bit_cast(bf8, ws[nw + 16 * i + c16][unit]);
+#pragma unroll
+            for (int part = 0; part < 3; part++) {
+                bf8 xb[WR];
+#pragma unroll
+                for (int q = 0; q < WR; q++) xb[q] = __builtin_bit_cast(bf8, xs[part][rw + 16 * q + c16][unit]);
+#pragma unroll
+                for (int q = 0; q < WR; q++)
+#pragma unroll
+                    for (int i = 0; i < WC; i++) {
+                        f4& s = part == 0 ? acc[i][q] : low[i][q];
+                        s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wa[i], xb[q], s, 0, 0, 0);
+                    }
+            }
+        }
+        if ((c & 1) || c + 1 == nchunks) {
+#pragma unroll
+            for (int i = 0; i < WC; i++)
+#pragma unroll
+                for (int q = 0; q < WR; q++) {
+                    const f4 t2 = tot[i][q] + acc[i][q];
+                    low[i][q] += acc[i][q] - (t2 - tot[i][q]);
+                    tot[i][q] = t2;
+                    acc[i][q] = f4{0.f, 0.f, 0.f, 0.f};
+                }
+        }
+        __syncthreads();
+    }
+    const bool vec = a.ldo % 4 == 0 && ((uintptr_t)a.out & 15u) == 0;
+    bool fin = true;
+#pragma unroll
+    for (int i = 0; i < WC; i++) {
+        const int n = n0 + nw + 16 * i + 4 * g;
+        f4 sc = {1.f, 1.f, 1.f, 1.f};
+        if constexpr (I8) {
+#pragma unroll
+            for (int e = 0; e < 4; e++) sc[e] = a.scale[min(n + e, a.n - 1)];
+        }
+#pragma unroll
+        for (int q = 0; q < WR; q++) {
+            const int r = r0 + rw + 16 * q + c16;
+            float* o = a.out + (int64_t)r * a.ldo + n;
+            f4 v = tot[i][q] + low[i][q];
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                if constexpr (I8) v[e] *= sc[e];
+                fin = fin && finite(v[e]);
+            }
+            if (r >= a.rows) continue;
+            if (vec && n + 3 < a.n) {
+                *reinterpret_cast<f4*>(o) = v;
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; e++)
+                    if (n + e < a.n) o[e] = v[e];
+            }
+        }
+    }
+    if (fin) return;
+    // this lane's outputs once more: those that are not finite are formed in k order
+#pragma unroll 1
+    for (int e = 0; e < WC * WR * 4; e++) {
+        const int n = n0 + nw + 16 * (e / (4 * WR)) + 4 * g + e % 4, r = r0 + rw + 16 * (e / 4 % WR) + c16;
+        if (n >= a.n || r >= a.rows) continue;
+        float* o = a.out + (int64_t)r * a.ldo + n;
+        if (!finite(*o)) *o = output_in_order<I8>(a, r, n);
+    }
+}
+
+template <int WR, int WC>
+hipError_t launch_tiled(const HeadArgs& a, hipStream_t stream) {
+    const int row_tiles = (a.rows + 32 * WR - 1) / (32 * WR);
+    const int tiles = row_tiles * ((a.n + 32 * WC - 1) / (32 * WC));
+    if (a.q)
+        hipLaunchKernelGGL((head_mfma_tiled_kernel<WR, WC, true>), dim3(xcd_grid(tiles)), dim3(kHT), 0, stream, a, row_tiles, tiles);
+    else
+        hipLaunchKernelGGL((head_mfma_tiled_kernel<WR, WC, false>), dim3(xcd_grid(tiles)), dim3(kHT), 0, stream, a, row_tiles, tiles);
     return hipGetLastError();
 }
 
@@ -454,11 +677,10 @@ __global__ __launch_bounds__(kHT) void head_pack_i8_kernel(int k, const uint16_t
     if (threadIdx.x == 0) scale[n] = scl;
 }
 
-// Rows are split into groups, one grid row each, so that the launch has about 2048 waves for the
-// chip's 1024 SIMDs; a group keeps at least two rows (the loads of one overlap the other's work).
-// Every group reads the weight again, from the last-level cache after the first.
-template <int KJ, int R>
-hipError_t launch_kr(HeadArgs a, hipStream_t stream) {
+// Rows are split into groups of at least two, one grid row each, while the launch has fewer than 2048
+// waves for the chip's 1024 SIMDs; every group reads the weight again.
+template <int KJ>
+hipError_t launch_k(HeadArgs a, hipStream_t stream) {
     const int tiles = (a.n + (kHT / 64) * R - 1) / ((kHT / 64) * R);
     const int waves = tiles * (kHT / 64);
     const int groups = std::max(1, std::min(2048 / waves, a.rows / 2));
@@ -466,35 +688,57 @@ hipError_t launch_kr(HeadArgs a, hipStream_t stream) {
     const dim3 grid(tiles, (a.rows + a.row_group - 1) / a.row_group);
     if (a.q) {
         if (a.k == 512 * KJ)
-            hipLaunchKernelGGL((head_i8_kernel<KJ, R, true>), grid, dim3(kHT), 0, stream, a);
+            hipLaunchKernelGGL((head_i8_kernel<KJ, true>), grid, dim3(kHT), 0, stream, a);
         else
-            hipLaunchKernelGGL((head_i8_kernel<KJ, R, false>), grid, dim3(kHT), 0, stream, a);
+            hipLaunchKernelGGL((head_i8_kernel<KJ, false>), grid, dim3(kHT), 0, stream, a);
     } else if (a.k == 512 * KJ) {
-        hipLaunchKernelGGL((head_kernel<KJ, R, true>), grid, dim3(kHT), 0, stream, a);
+        hipLaunchKernelGGL((head_kernel<KJ, true>), grid, dim3(kHT), 0, stream, a);
     } else {
-        hipLaunchKernelGGL((head_kernel<KJ, R, false>), grid, dim3(kHT), 0, stream, a);
+        hipLaunchKernelGGL((head_kernel<KJ, false>), grid, dim3(kHT), 0, stream, a);
     }
     return hipGetLastError();
+}
+
+// The matrix forms address a tile (at most 128 outputs, 64 rows) by 31-bit byte offsets.
+bool mfma_fits(const HeadArgs& a) {
+    constexpr int64_t kMax = int64_t(1) << 31;
+    return a.ldw < kMax / (128 * (a.q ? 1 : 2)) && a.ldx < kMax / (64 * 4);
 }
 
 }  // namespace
 
 hipError_t launch_head(const HeadArgs& a, hipStream_t stream) {
     if (a.rows <= 0 || a.n <= 0) return hipSuccess;
-    // The matrix-core form for 8 to 32 rows and at least 2560 outputs (160 or more workgroups of
-    // 16 outputs). Measured, 24 rows x 1024, matrix cores / VALU: 3072 outputs 6.8 / 7.9 us, 2048
-    // outputs 6.8 / 6.4 us; 8 rows x 3072 5.4 / 6.1 us; 64 rows (two row groups in turn) 13.4 /
-    // 12.6 us at 3072 outputs and 13.3 / 9.4 us at 2048.
-    if (a.rows >= 8 && a.rows <= 32 && a.n >= 2560 && a.k >= 64) return launch_mfma<1, 16>(a, stream);
-    // Outputs per wave: eight up to k = 1024 (four above, for registers); with one or two rows, two,
-    // so that the single pass over the weight is spread over four times as many waves.
-    const bool few = a.rows <= 2;
+    if (a.k <= 0 || a.k > 2048) return hipErrorInvalidValue;
+    // One to three rows (two above k = 1024) on the VALU: one pass over the weight with no operand to
+    // turn, 1 x 1024 -> 2048 2.5 us (split-K form 3.9), 3 x 1024 -> 2048 3.6 (3.9), but 4 x 1024 -> 3072
+    // 4.5 (4.1) and 3 x 2048 -> 3072 6.2 (5.0). (bf16, back to back, 6 weights in turn; int8 alike.)
+    const bool few = a.rows <= 2 || (a.rows == 3 && a.k <= 1024);
+    if (!few && mfma_fits(a)) {
+        // The split-K form with the smallest tile that leaves at most one workgroup per compute unit:
+        // its time is that of loading a tile (us, one round, k = 1024: 16 x 16 4.1, 16 x 32 4.5, 16 x 48
+        // 5.1, 32 x 48 7.5, 32 x 64 8.6, 32 x 96 10.3) and a second round adds the same again (32 x 48
+        // at 2 rounds 13.3). The two largest need k >= 512, as their eight waves take 64 k each
+        // (256 x 256 -> 3072: 32 x 96 6.7, tiled 5.3).
+        auto tiles = [&](int rt, int ct) { return (int64_t)((a.rows + 16 * rt - 1) / (16 * rt)) * ((a.n + 16 * ct - 1) / (16 * ct)); };
+        constexpr int kCUs = 256;
+        if (tiles(1, 1) <= kCUs) return launch_mfma<1, 1, 16>(a, stream);
+        if (tiles(1, 2) <= kCUs) return launch_mfma<1, 2, 8>(a, stream);
+        if (tiles(1, 3) <= kCUs) return launch_mfma<1, 3, 8>(a, stream);
+        if (tiles(2, 3) <= kCUs) return launch_mfma<2, 3, 8>(a, stream);
+        if (a.k >= 512 && tiles(2, 4) <= kCUs) return launch_mfma<2, 4, 8>(a, stream);
+        if (a.k >= 512 && tiles(2, 6) <= kCUs) return launch_mfma<2, 6, 8>(a, stream);
+        // The tiled form beyond: 64 x 128 tiles from one and a half workgroups per compute unit, else
+        // 32 x 64 (us, 32 x 64 / 64 x 128: 512 x 1024 -> 3072 18.6 / 23.9, 1024 x 1024 -> 3072 32.8 / 31.3,
+        // 2048 x 2048 -> 2048 85 / 61, 4096 x 1024 -> 3072 122 / 91; split-K 32 x 96: 19.5, 42, 95, 167).
+        if (2 * tiles(4, 8) >= 3 * kCUs) return launch_tiled<2, 4>(a, stream);
+        return launch_tiled<1, 2>(a, stream);
+    }
     switch ((a.k + 511) / 512) {
-        case 1: return few ? launch_kr<1, 2>(a, stream) : launch_kr<1, 8>(a, stream);
-        case 2: return few ? launch_kr<2, 2>(a, stream) : launch_kr<2, 8>(a, stream);
-        case 3: return few ? launch_kr<3, 2>(a, stream) : launch_kr<3, 4>(a, stream);
-        case 4: return few ? launch_kr<4, 2>(a, stream) : launch_kr<4, 4>(a, stream);
-        default: return hipErrorInvalidValue;
+        case 1: return launch_k<1>(a, stream);
+        case 2: return launch_k<2>(a, stream);
+        case 3: return launch_k<3>(a, stream);
+        default: return launch_k<4>(a, stream);
     }
 }
 
