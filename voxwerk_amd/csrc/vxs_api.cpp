@@ -74,6 +74,16 @@ struct HostBuf {
     }
 };
 
+// Workspace of the kernel that splits wide rows over several workgroups: allocated when first needed,
+// zeroed once (the kernel leaves its counters zero), used by one launch after the other on `stream`.
+struct SplitWs {
+    void* p = nullptr;
+    hipStream_t stream = nullptr;
+    hipEvent_t last = nullptr;  // recorded after its last launch (caller-supplied streams)
+    bool recorded = false;
+};
+constexpr int kSplitStreams = 4;  // caller-supplied streams a context holds a workspace for
+
 }  // namespace
 
 struct vxs_ctx {
@@ -93,6 +103,8 @@ struct vxs_ctx {
     HostBuf h_done;
     uint32_t done_seq = 0;  // wraps; the completion word is reset to seq - 1 before each launch
     void* noalloc = nullptr;  // this device's fixed scratch (vxs_sample_noalloc), looked up at create
+    SplitWs split_own;                  // for own_stream, which outlives every use
+    SplitWs split_ext[kSplitStreams];  // for streams set by the caller
 };
 
 struct vxs_history {
@@ -300,6 +312,68 @@ void set_resident(vxs::SampleArgs& a, const vxs_history* h, const int32_t* d_slo
     if (rng_stream >= 0) a.kflags |= vxs::KF_RNG | (rng_stream == 1 ? vxs::KF_RNG_SUB : 0u);
 }
 
+bool split_alloc(SplitWs& w, hipStream_t stream) {
+    if (w.p) return true;
+    // another thread may be capturing a graph: allocating is no part of that
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
+    bool ok = hipMalloc(&w.p, vxs::split_workspace_bytes()) == hipSuccess;
+    if (!ok) w.p = nullptr;
+    if (ok && hipMemsetAsync(w.p, 0, vxs::split_workspace_bytes(), stream) != hipSuccess) {
+        (void)hipFree(w.p);
+        w.p = nullptr;
+        ok = false;
+    }
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
+    if (!ok) (void)hipGetLastError();
+    return ok;
+}
+
+// The workspace a launch of `a` on the context's stream may use, or null (the call is not one that
+// splits, its stream is being captured, so that a replay could meet other launches in the workspace, or
+// none is free): the launch then takes one workgroup per row. A workspace belongs to one stream, in
+// whose order its launches run; one of a caller's streams may be destroyed and its handle used again, so
+// those launches record an event, and the workspace changes hands, or its next launch goes unordered,
+// only once that is complete.
+SplitWs* split_workspace(vxs_ctx* ctx, const vxs::SampleArgs& a) {
+    if (!vxs::split_wanted(a)) return nullptr;
+    hipStream_t st = ctx->stream;
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(st, &cap) != hipSuccess) {
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    if (cap != hipStreamCaptureStatusNone) return nullptr;
+    if (st == ctx->own_stream) return split_alloc(ctx->split_own, st) ? &ctx->split_own : nullptr;
+    auto idle = [](SplitWs& w) { return !w.recorded || hipEventQuery(w.last) == hipSuccess; };
+    SplitWs* w = nullptr;
+    for (SplitWs& x : ctx->split_ext)
+        if (x.p && x.stream == st) w = &x;
+    if (w) return idle(*w) || hipStreamWaitEvent(st, w->last, 0) == hipSuccess ? w : nullptr;
+    for (SplitWs& x : ctx->split_ext)
+        if (!w && idle(x)) w = &x;
+    if (!w) return nullptr;
+    if (!w->last && hipEventCreateWithFlags(&w->last, hipEventDisableTiming | hipEventDisableSystemFence) != hipSuccess) {
+        (void)hipGetLastError();
+        w->last = nullptr;
+        return nullptr;
+    }
+    if (!split_alloc(*w, st)) return nullptr;
+    w->stream = st;
+    return w;
+}
+
+// Enqueue the sampler on the context's stream.
+hipError_t launch(vxs_ctx* ctx, const vxs::SampleArgs& a) {
+    SplitWs* w = split_workspace(ctx, a);
+    hipError_t e = vxs::launch_sample(a, ctx->stream, w ? w->p : nullptr);
+    if (e == hipSuccess && w && w->last) {
+        e = hipEventRecord(w->last, ctx->stream);
+        w->recorded = true;
+    }
+    return e;
+}
+
 // Stage inputs and launch. On success the kernels are queued on ctx->stream.
 int stage_and_launch(vxs_ctx* ctx, int rows, int vocab, const float* logits, int64_t ld, const int32_t* hist_off,
                      const int32_t* hist_ids, const vxs_params* params, int params_stride, const double* u,
@@ -373,7 +447,7 @@ int stage_and_launch(vxs_ctx* ctx, int rows, int vocab, const float* logits, int
         a.direct_h1 = hist_off ? hoff[1] : 0;
         a.direct_u = u ? u[0] : 0.0;
     }
-    VXS_HIP(ctx, vxs::launch_sample(a, ctx->stream));
+    VXS_HIP(ctx, launch(ctx, a));
     return VXS_OK;
 }
 
@@ -545,6 +619,12 @@ VXS_API void vxs_destroy(vxs_ctx* ctx) {
     if (!ctx) return;
     (void)hipSetDevice(ctx->device);
     if (ctx->stream) (void)hipStreamSynchronize(ctx->stream);
+    if (ctx->split_own.p) (void)hipFree(ctx->split_own.p);
+    for (SplitWs& w : ctx->split_ext) {
+        if (w.recorded) (void)hipEventSynchronize(w.last);
+        if (w.last) (void)hipEventDestroy(w.last);
+        if (w.p) (void)hipFree(w.p);
+    }
     ctx->d_in.release();
     ctx->d_ids.release();
     ctx->d_draw.release();
@@ -722,7 +802,7 @@ VXS_API int vxs_sample_device(vxs_ctx* ctx, int rows, int vocab, const float* d_
         a.out_probs = d_out_probs;
         a.kflags = 0;
         a.path = choose_path(flags, rows, vocab);
-        VXS_HIP(ctx, vxs::launch_sample(a, ctx->stream));
+        VXS_HIP(ctx, launch(ctx, a));
         ctx->err.clear();
         return VXS_OK;
     } catch (...) {
@@ -761,7 +841,7 @@ VXS_API int vxs_sample_stats_device(vxs_ctx* ctx, int rows, int vocab, const flo
         a.out_stat_probs = d_probs;
         a.kflags = 0;
         a.path = choose_path(flags, rows, vocab);
-        VXS_HIP(ctx, vxs::launch_sample(a, ctx->stream));
+        VXS_HIP(ctx, launch(ctx, a));
         ctx->err.clear();
         return VXS_OK;
     } catch (...) {
@@ -1054,7 +1134,7 @@ VXS_API int vxs_sample_batch_device(vxs_ctx* ctx, vxs_history* h, int rows, int 
         a.kflags = 0;
         a.path = choose_path(flags, rows, vocab);
         set_resident(a, h, d_slots, append != 0, rng_stream_of(flags));
-        VXS_HIP(ctx, vxs::launch_sample(a, ctx->stream));
+        VXS_HIP(ctx, launch(ctx, a));
         ctx->err.clear();
         return VXS_OK;
     } catch (...) {

@@ -244,9 +244,14 @@ hipError_t noalloc_scratch(int device, void** out);
 // The lock a call holds while it uses `device`'s scratch (device as accepted by noalloc_scratch).
 std::mutex& noalloc_lock(int device);
 
-// Enqueue the sampler on `stream`. Returns hipSuccess or the launch error.
-hipError_t launch_sample(const SampleArgs& a, hipStream_t stream);
-hipError_t launch_sample_wide(const SampleArgs& a, hipStream_t stream);
+// Enqueue the sampler on `stream`. Returns hipSuccess or the launch error. split_ws: null, or a
+// workspace of split_workspace_bytes(), zero when first used and used by one launch after the other,
+// which wide rows of small batches are split with (split_wanted).
+hipError_t launch_sample(const SampleArgs& a, hipStream_t stream, void* split_ws = nullptr);
+hipError_t launch_sample_wide(const SampleArgs& a, hipStream_t stream, void* split_ws);
+constexpr int kSplitMaxRecords = 2048;  // rows x segments of one launch
+size_t split_workspace_bytes();
+bool split_wanted(const SampleArgs& a);
 // n successive NextDouble() of one generator into out[0..n) (one thread; a check and debug aid).
 hipError_t launch_draw_sequence(int32_t* state, int n, double* out, hipStream_t stream);
 

@@ -1,6 +1,9 @@
 // vxs_wide.hip — the sampler for vocabularies above 8192 (up to 2^19), one 256-thread workgroup
 // per row, streaming the row from HBM instead of holding it in registers.
 //
+// Calls whose rows are too few to fill the chip that way are split over several workgroups per row
+// (vxs_split.h, split_segment has the rule). The rest of this text is about one workgroup per row.
+//
 // One kernel (sample_wide_kernel), two algorithms. The ordered pass (wide_ordered_row) serves the
 // common sampled top-k rows in one read of the row; the general algorithm (wide_general_row) serves
 // every other row and the rows the ordered pass hands back, in the same workgroup, as follows.
@@ -24,6 +27,7 @@
 // kernels), ties at the cut resolved in index order, and an index-order draw; each step re-reads
 // the row (L2/HBM), so the general path costs several passes.
 #include <math.h>
+#include <stddef.h>
 #include <stdint.h>
 
 #include "vxs_device.h"
@@ -121,6 +125,21 @@ struct BlkW {
         for (int i = 0; i < kWW; i++) {
             const double x = __longlong_as_double((long long)s->slot[1][i]);
             base += i < wv ? x : 0.0;
+            tot += x;
+        }
+        __syncthreads();
+        total = tot;
+        return base + incl - v;
+    }
+    __device__ __forceinline__ uint64_t excl(uint64_t v, uint64_t& total) const {
+        const uint64_t incl = wave_incl_sum(v);
+        if (lane == 0) s->slot[1][wv] = readlane64(incl, 63);
+        __syncthreads();
+        uint64_t base = 0, tot = 0;
+#pragma unroll
+        for (int i = 0; i < kWW; i++) {
+            const uint64_t x = s->slot[1][i];
+            base += i < wv ? x : 0;
             tot += x;
         }
         __syncthreads();
@@ -898,6 +917,174 @@ __device__ __forceinline__ float x_threshold(float tau, float invT) {
     return key2f(k);
 }
 
+// The tail of a row whose candidates the four waves hold in registers, in index order (wave ranges
+// ascending, slot lane + 64 q of a wave): kk the keys of the exact values (0: no entry), ii the indices,
+// [klo, khi] the workgroup's smallest and largest key, at most K ties aside at or above the k-th
+// largest. `worker` marks the wave that runs the sequential part. Returns true, before anything was
+// written, when more candidates tie at the k-th largest than the exact regime holds.
+__device__ __forceinline__ bool ordered_tail(const SampleArgs& a, int vec, int r, const vxs_params& P, const RowX& X, BlkW& g,
+                                             WideSmem& s, const uint32_t (&kk)[kPerL], const int32_t (&ii)[kPerL],
+                                             uint32_t klo, uint32_t khi, int K, bool topk_on, bool worker, float* orow,
+                                             double* prow, const float* __restrict__ xrow) {
+    const int V = a.vocab;
+    // ---- all waves: the k-th largest of the buffered keys, the maximum, the candidates
+    const uint32_t kthkey = topk_on ? block_kth_radix(kk, klo, khi, K, s.h.h3, g.t, g.lane) : 1u;
+    const float mx = key2f(khi);
+    // the candidates (keys >= the k-th largest; 0 < 1 <= every valid key) in index order: the
+    // waves' counts, then each wave writes its own after those of the waves before it
+    {
+        uint32_t mine = 0;
+#pragma unroll
+        for (int q = 0; q < kPerL; q++) mine += (uint32_t)__builtin_popcountll(__ballot(kk[q] >= kthkey));
+        if (g.lane == 0) s.wcand[g.wv] = (int32_t)mine;
+    }
+    __syncthreads();
+    int n = 0, off = 0;
+#pragma unroll
+    for (int w = 0; w < kWW; w++) {
+        off += w < g.wv ? s.wcand[w] : 0;
+        n += s.wcand[w];
+    }
+    if (n > kCandW) return true;  // ties beyond the exact-regime capacity: the general algorithm
+    // (d, index) keys, d = v - max, over the wave buffers (every wave has read its own into registers)
+    uint64_t* ckey = reinterpret_cast<uint64_t*>(&s.wkey[0][0]);
+    {
+        uint32_t m = (uint32_t)off;
+#pragma unroll
+        for (int q = 0; q < kPerL; q++) {
+            const bool keep = kk[q] >= kthkey;
+            const uint64_t bal = __ballot(keep);
+            if (keep) {
+                const uint32_t pos = m + __builtin_amdgcn_mbcnt_hi((uint32_t)(bal >> 32),
+                                                                   __builtin_amdgcn_mbcnt_lo((uint32_t)bal, 0u));
+                const float v = key2f(kk[q]);
+                s.ex.cx[pos] = v;
+                s.ex.ci[pos] = ii[q];
+                ckey[pos] = ((uint64_t)f2key(v - mx) << 32) | (uint32_t)ii[q];
+            }
+            m += (uint32_t)__builtin_popcountll(bal);
+        }
+        if (g.t < 8) ckey[n + g.t] = ~0ull;  // above every key: the rank loop reads whole groups of eight
+    }
+    const float kth = topk_on ? key2f(kthkey) : kNegInf;
+    if (orow) for_row(xrow, V, vec, g.t, X, [&](int i, float x) { orow[i] = x < kth ? kNegInf : x; });
+    if (prow)
+        for (int i = g.t; i < V; i += kTW) prow[i] = 0.0;
+    __syncthreads();
+
+    __builtin_amdgcn_s_setprio(0);
+    // ---- all waves: thread t holds candidate t (index order); its position in (d, index) order,
+    // counted over the keys eight at a time, and its exp(d)                        Sampler.cs:57
+    if (g.t < n) {
+        const uint64_t kt = ckey[g.t];
+        typedef unsigned long long u64x2 __attribute__((ext_vector_type(2)));
+        const u64x2* kp = reinterpret_cast<const u64x2*>(ckey);
+        auto below = [&](const u64x2 (&q)[4]) {
+            int c = 0;
+#pragma unroll
+            for (int k = 0; k < 4; k++) c += (q[k].x < kt ? 1 : 0) + (q[k].y < kt ? 1 : 0);
+            return c;
+        };
+        // the next group's reads are issued before the current group is counted
+        u64x2 ga[4], gb[4];
+#pragma unroll
+        for (int k = 0; k < 4; k++) ga[k] = kp[k];
+        int po = 0, l = 8;
+        for (; l + 8 < n; l += 16) {
+#pragma unroll
+            for (int k = 0; k < 4; k++) gb[k] = kp[l / 2 + k];
+            po += below(ga);
+#pragma unroll
+            for (int k = 0; k < 4; k++) ga[k] = kp[l / 2 + 4 + k];
+            po += below(gb);
+        }
+        if (l < n) {
+#pragma unroll
+            for (int k = 0; k < 4; k++) gb[k] = kp[l / 2 + k];
+            po += below(ga);
+#pragma unroll
+            for (int k = 0; k < 4; k++) ga[k] = gb[k];
+        }
+        po += below(ga);
+        s.ex.cs[po] = (int16_t)g.t;
+        s.ex.cp[g.t] = exp((double)(s.ex.cx[g.t] - mx));
+    }
+    __syncthreads();
+    if (!worker) return false;
+
+    // ---- the worker wave: the reference's fp64 arithmetic on the candidates in index order
+    double* cp = s.ex.cp;
+    const double sum = seq_sum_pipe(cp, n);  // sequential in index order              :58
+    for (int j = g.lane; j < n; j += 64) cp[j] = cp[j] / sum;  //                         :60
+    wave_sync();
+    if (P.top_p < 1.0f) {  //                                                          :62-75
+        bool ok = true;
+        for (int q = g.lane; q < n - 1; q += 64) {
+            const int a0 = s.ex.cs[q], b0 = s.ex.cs[q + 1];
+            const double pa = cp[a0], pb = cp[b0];
+            ok = ok && (pa < pb || (pa == pb && a0 < b0));
+        }
+        if (__ballot(!ok)) {  // rank by (p, index) directly
+            int rk[kCandW / 64];
+#pragma unroll
+            for (int k = 0; k < kCandW / 64; k++) {
+                const int j = g.lane + 64 * k;
+                rk[k] = j < n ? seq_rank(cp, n, j) : 0;
+            }
+            wave_sync();
+#pragma unroll
+            for (int k = 0; k < kCandW / 64; k++) {
+                const int j = g.lane + 64 * k;
+                if (j < n) s.ex.cs[rk[k]] = (int16_t)j;
+            }
+            wave_sync();
+        }
+        // the last sorted position is never removed (the reference's loop runs j < n - 1)
+        double* ps = reinterpret_cast<double*>(&s.widx[0][0]);  // p in (p, index) order
+        for (int q = g.lane; q < n; q += 64) ps[q] = cp[s.ex.cs[q]];
+        wave_sync();
+        const int nrem = wave_topp_cut_par(ps, n, (double)(1.0f - P.top_p), g.lane);
+        for (int q = g.lane; q < nrem; q += 64) cp[s.ex.cs[q]] = 0.0;
+        wave_sync();
+        // The entries left with p > 0 (or NaN), in index order: the second sum and the draw over
+        // them alone are the reference's over all n (adding zero changes no sum; the draw skips
+        // p <= 0).
+        double* kp = ps;  // the sorted copy is no longer needed
+        int32_t* kid = &s.widx[2][0];
+        int nk = 0;
+        for (int b = 0; b < n; b += 64) {
+            const int j = b + g.lane;
+            const double pj = j < n ? cp[j] : 0.0;
+            const bool keep = j < n && !(pj <= 0.0);
+            const uint64_t bal = __ballot(keep);
+            if (keep) {
+                const int pos = nk + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(bal >> 32),
+                                                                    __builtin_amdgcn_mbcnt_lo((uint32_t)bal, 0u));
+                kp[pos] = pj;
+                kid[pos] = s.ex.ci[j];
+            }
+            nk += __builtin_popcountll(bal);
+        }
+        wave_sync();
+        const double s2 = seq_sum(kp, nk);  // probs.Sum() in index order               :73
+        for (int q = g.lane; q < nk; q += 64) kp[q] = kp[q] / s2;  //                  :74
+        if (prow)
+            for (int j = g.lane; j < n; j += 64) cp[j] = cp[j] / s2;
+        wave_sync();
+        const double u = row_uniform(a, r);
+        const int pick = wave_draw(kp, kid, nk, u);  // inverse-CDF draw in index order :77-87
+        if (g.lane == 0) put_id(a, r, pick);
+    } else {
+        const double u = row_uniform(a, r);
+        const int pick = wave_draw(cp, s.ex.ci, n, u);  // inverse-CDF draw in index order :77-87
+        if (g.lane == 0) put_id(a, r, pick);
+    }
+    if (prow)
+        for (int j = g.lane; j < n; j += 64) prow[s.ex.ci[j]] = cp[j];
+    return false;
+}
+
+
 // =====================================================================================
 // The ordered pass: the rows row_ordered() selects, in one read of the row. Returns true when the
 // general algorithm must serve the row instead.
@@ -1247,161 +1434,7 @@ __device__ __forceinline__ bool wide_ordered_row(const SampleArgs& a, int vec, i
         for (int w = 0; w < kWW; w++) nw += s.wslot[w];
         if (nw == 1) worker = s.wslot[g.wv] != 0;
     }
-    // ---- all waves: the k-th largest of the buffered keys, the maximum, the candidates
-    const uint32_t kthkey = topk_on ? block_kth_radix(kk, klo, khi, K, s.h.h3, g.t, g.lane) : 1u;
-    const float mx = key2f(khi);
-    // the candidates (keys >= the k-th largest; 0 < 1 <= every valid key) in index order: the
-    // waves' counts, then each wave writes its own after those of the waves before it
-    {
-        uint32_t mine = 0;
-#pragma unroll
-        for (int q = 0; q < kPerL; q++) mine += (uint32_t)__builtin_popcountll(__ballot(kk[q] >= kthkey));
-        if (g.lane == 0) s.wcand[g.wv] = (int32_t)mine;
-    }
-    __syncthreads();
-    int n = 0, off = 0;
-#pragma unroll
-    for (int w = 0; w < kWW; w++) {
-        off += w < g.wv ? s.wcand[w] : 0;
-        n += s.wcand[w];
-    }
-    if (n > kCandW) return true;  // ties beyond the exact-regime capacity: the general algorithm
-    // (d, index) keys, d = v - max, over the wave buffers (every wave has read its own into registers)
-    uint64_t* ckey = reinterpret_cast<uint64_t*>(&s.wkey[0][0]);
-    {
-        uint32_t m = (uint32_t)off;
-#pragma unroll
-        for (int q = 0; q < kPerL; q++) {
-            const bool keep = kk[q] >= kthkey;
-            const uint64_t bal = __ballot(keep);
-            if (keep) {
-                const uint32_t pos = m + __builtin_amdgcn_mbcnt_hi((uint32_t)(bal >> 32),
-                                                                   __builtin_amdgcn_mbcnt_lo((uint32_t)bal, 0u));
-                const float v = key2f(kk[q]);
-                s.ex.cx[pos] = v;
-                s.ex.ci[pos] = ii[q];
-                ckey[pos] = ((uint64_t)f2key(v - mx) << 32) | (uint32_t)ii[q];
-            }
-            m += (uint32_t)__builtin_popcountll(bal);
-        }
-        if (g.t < 8) ckey[n + g.t] = ~0ull;  // above every key: the rank loop reads whole groups of eight
-    }
-    const float kth = topk_on ? key2f(kthkey) : kNegInf;
-    if (orow) for_row(xrow, V, vec, g.t, X, [&](int i, float x) { orow[i] = x < kth ? kNegInf : x; });
-    if (prow)
-        for (int i = g.t; i < V; i += kTW) prow[i] = 0.0;
-    __syncthreads();
-
-    __builtin_amdgcn_s_setprio(0);
-    // ---- all waves: thread t holds candidate t (index order); its position in (d, index) order,
-    // counted over the keys eight at a time, and its exp(d)                        Sampler.cs:57
-    if (g.t < n) {
-        const uint64_t kt = ckey[g.t];
-        typedef unsigned long long u64x2 __attribute__((ext_vector_type(2)));
-        const u64x2* kp = reinterpret_cast<const u64x2*>(ckey);
-        auto below = [&](const u64x2 (&q)[4]) {
-            int c = 0;
-#pragma unroll
-            for (int k = 0; k < 4; k++) c += (q[k].x < kt ? 1 : 0) + (q[k].y < kt ? 1 : 0);
-            return c;
-        };
-        // the next group's reads are issued before the current group is counted
-        u64x2 ga[4], gb[4];
-#pragma unroll
-        for (int k = 0; k < 4; k++) ga[k] = kp[k];
-        int po = 0, l = 8;
-        for (; l + 8 < n; l += 16) {
-#pragma unroll
-            for (int k = 0; k < 4; k++) gb[k] = kp[l / 2 + k];
-            po += below(ga);
-#pragma unroll
-            for (int k = 0; k < 4; k++) ga[k] = kp[l / 2 + 4 + k];
-            po += below(gb);
-        }
-        if (l < n) {
-#pragma unroll
-            for (int k = 0; k < 4; k++) gb[k] = kp[l / 2 + k];
-            po += below(ga);
-#pragma unroll
-            for (int k = 0; k < 4; k++) ga[k] = gb[k];
-        }
-        po += below(ga);
-        s.ex.cs[po] = (int16_t)g.t;
-        s.ex.cp[g.t] = exp((double)(s.ex.cx[g.t] - mx));
-    }
-    __syncthreads();
-    if (!worker) return false;
-
-    // ---- the worker wave: the reference's fp64 arithmetic on the candidates in index order
-    double* cp = s.ex.cp;
-    const double sum = seq_sum_pipe(cp, n);  // sequential in index order              :58
-    for (int j = g.lane; j < n; j += 64) cp[j] = cp[j] / sum;  //                         :60
-    wave_sync();
-    if (P.top_p < 1.0f) {  //                                                          :62-75
-        bool ok = true;
-        for (int q = g.lane; q < n - 1; q += 64) {
-            const int a0 = s.ex.cs[q], b0 = s.ex.cs[q + 1];
-            const double pa = cp[a0], pb = cp[b0];
-            ok = ok && (pa < pb || (pa == pb && a0 < b0));
-        }
-        if (__ballot(!ok)) {  // rank by (p, index) directly
-            int rk[kCandW / 64];
-#pragma unroll
-            for (int k = 0; k < kCandW / 64; k++) {
-                const int j = g.lane + 64 * k;
-                rk[k] = j < n ? seq_rank(cp, n, j) : 0;
-            }
-            wave_sync();
-#pragma unroll
-            for (int k = 0; k < kCandW / 64; k++) {
-                const int j = g.lane + 64 * k;
-                if (j < n) s.ex.cs[rk[k]] = (int16_t)j;
-            }
-            wave_sync();
-        }
-        // the last sorted position is never removed (the reference's loop runs j < n - 1)
-        double* ps = reinterpret_cast<double*>(&s.widx[0][0]);  // p in (p, index) order
-        for (int q = g.lane; q < n; q += 64) ps[q] = cp[s.ex.cs[q]];
-        wave_sync();
-        const int nrem = wave_topp_cut_par(ps, n, (double)(1.0f - P.top_p), g.lane);
-        for (int q = g.lane; q < nrem; q += 64) cp[s.ex.cs[q]] = 0.0;
-        wave_sync();
-        // The entries left with p > 0 (or NaN), in index order: the second sum and the draw over
-        // them alone are the reference's over all n (adding zero changes no sum; the draw skips
-        // p <= 0).
-        double* kp = ps;  // the sorted copy is no longer needed
-        int32_t* kid = &s.widx[2][0];
-        int nk = 0;
-        for (int b = 0; b < n; b += 64) {
-            const int j = b + g.lane;
-            const double pj = j < n ? cp[j] : 0.0;
-            const bool keep = j < n && !(pj <= 0.0);
-            const uint64_t bal = __ballot(keep);
-            if (keep) {
-                const int pos = nk + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(bal >> 32),
-                                                                    __builtin_amdgcn_mbcnt_lo((uint32_t)bal, 0u));
-                kp[pos] = pj;
-                kid[pos] = s.ex.ci[j];
-            }
-            nk += __builtin_popcountll(bal);
-        }
-        wave_sync();
-        const double s2 = seq_sum(kp, nk);  // probs.Sum() in index order               :73
-        for (int q = g.lane; q < nk; q += 64) kp[q] = kp[q] / s2;  //                  :74
-        if (prow)
-            for (int j = g.lane; j < n; j += 64) cp[j] = cp[j] / s2;
-        wave_sync();
-        const double u = row_uniform(a, r);
-        const int pick = wave_draw(kp, kid, nk, u);  // inverse-CDF draw in index order :77-87
-        if (g.lane == 0) put_id(a, r, pick);
-    } else {
-        const double u = row_uniform(a, r);
-        const int pick = wave_draw(cp, s.ex.ci, n, u);  // inverse-CDF draw in index order :77-87
-        if (g.lane == 0) put_id(a, r, pick);
-    }
-    if (prow)
-        for (int j = g.lane; j < n; j += 64) prow[s.ex.ci[j]] = cp[j];
-    return false;
+    return ordered_tail(a, vec, r, P, X, g, s, kk, ii, klo, khi, K, topk_on, worker, orow, prow, xrow);
 }
 
 // One workgroup per row: the ordered pass when the row's options allow it, else (or when that pass
@@ -1421,13 +1454,47 @@ __global__ __launch_bounds__(kTW) __attribute__((amdgpu_waves_per_eu(4))) void s
     wide_general_row(a, vec, r, g, s, bm_dyn);
 }
 
+#include "vxs_split.h"
+
 }  // namespace
 
-hipError_t launch_sample_wide(const SampleArgs& a, hipStream_t stream) {
+size_t split_workspace_bytes() { return (sizeof(SplitRow) + sizeof(SplitSeg)) * (size_t)kSplitMaxRecords; }
+
+// Rows over several workgroups (vxs_split.h): the sweeps of 1024 entries per segment, 0 when the call is not
+// for it. Segments of 4096 entries while the call then has at most 1024 of them (four workgroups per
+// compute unit, all resident), else of 10240; one workgroup per row when the call writes back, or has
+// rows enough to keep the compute units busy that way (us, split / one workgroup per row, top-k 50 or as
+// said: 1 x 151936 19.9 / 74, 16 x 151936 23.8 / 73, 64 32.8 / 78, 136 51.3 / 79, 200 x 20000 26.6 / 28.4,
+// 300 x 20000 31.8 / 29.9, 128 x 151936 at top-k 200 70 / 86; nucleus, top-p 0.9: 4 x 151936 25.6 / 1017, 64
+// 45.7 / 1361, 128 82 / 1385, 300 x 20000 40.7 / 220).
+static int split_segment(const SampleArgs& a) {
+    if (a.rows > 192 || a.out_logits || a.out_probs || (a.kflags & KF_STOP_AFTER_PENALTY)) return 0;
+    for (int nc : {4, 10}) {
+        const int len = 1024 * nc, S = (a.vocab + len - 1) / len;
+        if (S <= kSplitMaxSegs && (int64_t)a.rows * S <= (nc == 4 ? 1024 : kSplitMaxRecords)) return nc;
+    }
+    return 0;
+}
+
+bool split_wanted(const SampleArgs& a) { return a.vocab > kRowResidentMaxVocab && split_segment(a) != 0; }
+
+hipError_t launch_sample_wide(const SampleArgs& a, hipStream_t stream, void* split_ws) {
     if (a.rows <= 0) return hipSuccess;
     if (a.vocab <= 0 || a.vocab > kWideMaxVocab) return hipErrorNotSupported;
     const int vec = (a.ld % 4 == 0) && (((uintptr_t)a.logits & 15u) == 0) ? 1 : 0;
-    const size_t dyn = sizeof(uint32_t) * (size_t)((a.vocab + 31) / 32 + kBmPad);
+    size_t dyn = sizeof(uint32_t) * (size_t)((a.vocab + 31) / 32 + kBmPad);
+    const int nc = split_ws ? split_segment(a) : 0;
+    if (nc) {
+        const int S = (a.vocab + 1024 * nc - 1) / (1024 * nc);
+        SplitRow* rows = static_cast<SplitRow*>(split_ws);
+        SplitSeg* segs = reinterpret_cast<SplitSeg*>(rows + kSplitMaxRecords);
+        dyn = dyn < 128u * nc ? 128u * nc : dyn;  // a segment's bitmap may be longer than a short row's
+        if (nc == 4)
+            hipLaunchKernelGGL(sample_split_kernel<4>, dim3(a.rows * S), dim3(kTW), dyn, stream, a, vec, S, rows, segs);
+        else
+            hipLaunchKernelGGL(sample_split_kernel<10>, dim3(a.rows * S), dim3(kTW), dyn, stream, a, vec, S, rows, segs);
+        return hipGetLastError();
+    }
     hipLaunchKernelGGL(sample_wide_kernel, dim3(a.rows), dim3(kTW), dyn, stream, a, vec);
     return hipGetLastError();
 }
