@@ -76,7 +76,7 @@ def test_split_nucleus_ties_and_cuts(ctx, vocab):
     x[9] = np.linspace(0, -1e-3, vocab)
     x[10, : vocab // 2] = -np.inf
     for top_p in (0.95, 0.5, 0.05, 1.0):
-        for k in (0, 50, 256):
+        for k in (0, 50, 256, 300, vocab // 3):
             p = options(rng, rows, vocab, top_p=np.float32(top_p), top_k=k, rep_penalty=np.float32(1.0), temperature=np.float32(1.0))
             for u in (rng.random(rows), np.full(rows, 0.0), np.full(rows, 1.0 - 2.0**-53)):
                 check(ctx, x, p, u, label=f"ties V={vocab} p={top_p} k={k}")

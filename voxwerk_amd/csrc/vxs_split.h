@@ -20,7 +20,8 @@
 // three per unit took 47.6 to 61 us.
 //
 // Masses are the fixed-point ones of the other kernels (multiples of 2^-F, exact sums in any order).
-// Rows that none of this fits (top-k above 256, more ties than the exact regime or a list holds, top-p
+// A top-k above 256 goes through the same stages over counts first, to its k-th largest value, and then on
+// as a nucleus row over what is left. Rows that none of this fits (more ties than the exact regime or a list holds, top-p
 // not above 0) are sampled by the last workgroup to leave, with the general algorithm.
 //
 // A meeting is a bounded wait: workgroups are dispatched in order, so a row's arrive together unless
@@ -40,9 +41,10 @@ constexpr uint64_t kMeetTicks = 50000;                  // 500 us of the 100 MHz
 constexpr uint32_t kAbandoned = 0x80000000u;
 
 struct alignas(64) SplitRow {  // zero between calls
-    uint32_t meet[4];
+    uint32_t meet[8];
     uint32_t left;
-    alignas(64) uint64_t coarse[kCoarse], sub[kSub];  // the row's masses, summed up by its segments
+    // the row's counts (top-k above kKMax) and masses, summed up by its segments
+    alignas(64) uint64_t coarse[2][kCoarse], sub[2][kSub];
 };
 struct alignas(16) SplitSeg {
     uint32_t maxkey, cnt, bad, n;     // largest key; finite entries; 1 non-finite, 2 bad history id; entries listed
@@ -487,8 +489,7 @@ __device__ __forceinline__ SplitEnd split_row(const SampleArgs& a, int vec, int 
     {
         const float wmx = wave_fmax(tmx);
         if (g.lane == 0) s.slot[2][g.wv] = f2key(wmx);
-        if (topp)
-            for (int i = g.t; i < kFineMass; i += kTW) lds64[i] = 0;
+        for (int i = g.t; i < kFineMass; i += kTW) lds64[i] = 0;
         __syncthreads();
         if (g.t == 0) {
             put(me.maxkey, max(max((uint32_t)s.slot[2][0], (uint32_t)s.slot[2][1]), max((uint32_t)s.slot[2][2], (uint32_t)s.slot[2][3])));
@@ -499,6 +500,7 @@ __device__ __forceinline__ SplitEnd split_row(const SampleArgs& a, int vec, int 
     const bool in = g.lane < S;  // lane l of every wave reads segment l's record
     if (!meet(&row.meet[0], S, g, s)) return kEndUnsampled;
     float mx;
+    bool count_first;  // top-k above kKMax: the k-th largest first, by the same stages over counts
     {
         const uint32_t flags = in ? get(segs[g.lane].bad) : 0u;
         const uint32_t rcnt = wave_sum(in ? get(segs[g.lane].cnt) : 0u);
@@ -508,7 +510,7 @@ __device__ __forceinline__ SplitEnd split_row(const SampleArgs& a, int vec, int 
             if (seg == 0 && g.t == 0) put_id(a, r, bid ? VXS_ERR_ID_OUT_OF_RANGE : nf ? VXS_ERR_NONFINITE : V - 1);
             return kEndLeave;
         }
-        if (K > 0 && K < V && (uint32_t)K < rcnt) return kEndUnsampled;  // top-k above kKMax
+        count_first = K > 0 && K < V && (uint32_t)K < rcnt;
     }
     const double thr = (double)(1.0f - P.top_p);
     if (topp && !(thr < 1.0)) return kEndUnsampled;
@@ -520,6 +522,10 @@ __device__ __forceinline__ SplitEnd split_row(const SampleArgs& a, int vec, int 
     auto units = [&](float q) -> uint64_t {
         asm volatile("" : "+v"(q));  // formed where it is used: 64 bits per entry are not kept
         return (uint64_t)__double_as_longlong((double)q + unit) - (uint64_t)__double_as_longlong(unit);
+    };
+    auto part_of = [](float q) -> uint32_t {
+        asm volatile("" : "+v"(q));  // (the same)
+        return __float_as_uint(q) >> 14;
     };
     const uint32_t base17 = (uint32_t)(127 - F) << 6;  // bits >> 17 of the smallest mass, 2^-F
 #pragma unroll
@@ -533,213 +539,10 @@ __device__ __forceinline__ SplitEnd split_row(const SampleArgs& a, int vec, int 
     uint32_t cidx = 0;
     bool tied = false;        // all of the cut's part have one key
     int own_n = 0;            // this segment's entries of the part
-    double kept_l;            // lane l: the kept mass of segment l
-    if (topp) {
-#pragma unroll
-        for (int e = 0; e < NE; e++) {
-            if (e % 4 == 0) __builtin_amdgcn_sched_barrier(0);
-            const uint32_t b = __float_as_uint(v[e]);
-            if (b) atomicAdd((unsigned long long*)&lds64[(b >> 17) - base17], (unsigned long long)units(v[e]));
-        }
-        __syncthreads();
-        uint64_t own = 0;  // thread t: this segment's mass in bucket t
-        if (g.t < kCoarse) {
-#pragma unroll
-            for (int i = 0; i < 16; i++) own += lds64[16 * g.t + ((i + g.t) & 15)];
-            if (own) sum_up(row.coarse[g.t], own);
-        }
-        if (!meet(&row.meet[1], S, g, s)) return kEndUnsampled;
-        // the bucket where the ascending cumulative mass crosses T
-        auto crossing = [&](uint64_t h, double rest, double& below, double& total) -> int {
-            const double run = g.excl((double)h, total);
-            const double t0 = rest >= 0.0 ? rest : floor(thr * total);  // (negative: T itself is sought)
-            if (h != 0 && run <= t0 && t0 - run < (double)h) {
-                s.wcand[0] = g.t;
-                s.slot[2][0] = (uint64_t)__double_as_longlong(run);
-            }
-            __syncthreads();
-            total = readlane_d(total, 0);  // (uniform: in scalar registers from here)
-            below = readlane_d(__longlong_as_double((long long)s.slot[2][0]), 0);
-            return __builtin_amdgcn_readfirstlane(s.wcand[0]);
-        };
-        uint64_t h = g.t < kCoarse ? get(row.coarse[g.t]) : 0ull;
-        double below, total;
-        const int bc = crossing(h, -1.0, below, total);
-        const double T = floor(thr * total);
-        if (T >= total) return kEndUnsampled;  // top-p so small that only the last entry stays
-        double kept = readlane_d(g.dsum(g.t > bc ? (double)own : 0.0), 0);  // this segment's mass above the bucket
-        // its 128 parts
-        if (g.t < kSub) lds64[g.t] = 0;
-        __syncthreads();
-        const uint32_t q21 = (uint32_t)bc + (base17 >> 4);
-#pragma unroll
-        for (int e = 0; e < NE; e++) {
-            const uint32_t b = __float_as_uint(v[e]);
-            if ((b >> 21) == q21) atomicAdd((unsigned long long*)&lds64[(b >> 14) & (kSub - 1)], (unsigned long long)units(v[e]));
-        }
-        __syncthreads();
-        own = g.t < kSub ? lds64[g.t] : 0;
-        if (own) sum_up(row.sub[g.t], own);
-        if (!meet(&row.meet[2], S, g, s)) return kEndUnsampled;
-        h = g.t < kSub ? get(row.sub[g.t]) : 0ull;
-        double sub_below, sub_total;
-        const int bf = crossing(h, T - below, sub_below, sub_total);
-        below += sub_below;
-        qcut = (q21 << 7) + (uint32_t)bf;
-        kept += readlane_d(g.dsum(g.t > bf ? (double)own : 0.0), 0);
-        // the part's entries as (d, index) keys: their indices first, then their values read again, all at
-        // once (few: one each per thread)
-        if (g.t == 0) s.n = 0;
-        int32_t* mine = reinterpret_cast<int32_t*>(lds64 + kSub);  // indices of this segment's entries of the part
-        __syncthreads();
-#pragma unroll
-        for (int e = 0; e < NE; e++)
-            if ((__float_as_uint(v[e]) >> 14) == qcut) mine[atomicAdd(&s.n, 1) & (kMine - 1)] = lo + 1024 * (e / 4) + 4 * g.t + (e & 3);
-        __syncthreads();
-        uint32_t kmin = 0xffffffffu, kmax = 0;
-        own_n = __builtin_amdgcn_readfirstlane(s.n);
-        if (own_n <= kMine) {
-            for (int j = g.t; j < own_n; j += kTW) {
-                const int i = mine[j];
-                const uint32_t key = f2key(X(i, xrow[i]) - mx);
-                kmin = min(kmin, key);
-                kmax = max(kmax, key);
-                if (j < kSegPart) put(me.part[j], ((uint64_t)key << 32) | (uint32_t)i);
-            }
-        } else {  // many: ties, most likely; each thread reads its own
-#pragma unroll 4
-            for (int e = 0; e < NE; e++) {
-                const int i = lo + 1024 * (e / 4) + 4 * g.t + (e & 3);
-                bool in_part = false;
-#pragma unroll
-                for (int q = 0; q < NE; q++) in_part |= q == e && (__float_as_uint(v[q]) >> 14) == qcut;
-                const uint32_t key = in_part ? f2key(X(i, xrow[i]) - mx) : 0u;
-                kmin = in_part ? min(kmin, key) : kmin;
-                kmax = max(kmax, key);
-            }
-        }
-        kmin = g.umin(kmin);
-        kmax = g.umax(kmax);
-        if (g.t == 0) {
-            put(me.n, (uint32_t)own_n);
-            put(me.kmin, kmin);
-            put(me.kmax, kmax);
-            put(me.kept, (uint64_t)kept);
-        }
-        if (!meet(&row.meet[3], S, g, s)) return kEndUnsampled;
-        const uint32_t n_l = in ? get(segs[g.lane].n) : 0u;
-        const uint32_t n = wave_sum(n_l);
-        kept_l = in ? (double)get(segs[g.lane].kept) : 0.0;
-        kmin = wave_umin(in ? get(segs[g.lane].kmin) : 0xffffffffu);
-        kmax = wave_umax(in ? get(segs[g.lane].kmax) : 0u);
-        tied = kmin == kmax;
-        if (tied) {
-            // one key (ties, or one entry): the crossing follows index order among them
-            const double w = (double)units(mass_of(exp_neg(key2f(kmin)), Cb));
-            const uint32_t nth = (uint32_t)((T - below) / w);  // entries of the part that go (exact integers)
-            const uint32_t before = wave_incl_sum(n_l) - n_l;
-            const uint32_t go_l = min(n_l, nth > before ? nth - before : 0u);
-            kept_l += w * (double)(n_l - go_l);
-            ckey = kmin;
-            const uint32_t go = readlane(go_l, seg);  // this segment's first `go` tied entries in index order go
-            cidx = 0;
-            if (go == (uint32_t)own_n) {
-                cidx = 0x7fffffffu;
-            } else if (go) {  // uniform: the index of entry number `go` among them
-                uint32_t run = 0;
-#pragma unroll 1
-                for (int c = 0; c < NC; c++) {
-                    uint32_t m4 = 0;
-#pragma unroll
-                    for (int e = 0; e < NE; e++)
-                        if (e / 4 == c) m4 |= (__float_as_uint(v[e]) >> 14) == qcut ? 1u << (e & 3) : 0u;
-                    uint32_t t4;
-                    const uint32_t ex = run + g.excl((uint32_t)__builtin_popcount(m4), t4);
-                    if (go >= ex && go < ex + (uint32_t)__builtin_popcount(m4)) {
-                        for (uint32_t k = go - ex; k; k--) m4 &= m4 - 1;
-                        s.wcand[1] = lo + 1024 * c + 4 * g.t + __builtin_ctz(m4);
-                    }
-                    run += t4;
-                }
-                __syncthreads();
-                cidx = (uint32_t)s.wcand[1];
-            }
-        } else if (n > (uint32_t)kRowPart || __ballot(n_l > (uint32_t)kSegPart)) {
-            return kEndUnsampled;
-        } else {
-            uint64_t* list = lds64;                   // [n] keys
-            uint64_t* mass = lds64 + kRowPart;        // [n] their masses
-            uint64_t* kept_s = lds64 + 2 * kRowPart;  // [S]
-            uint32_t* before = reinterpret_cast<uint32_t*>(kept_s + kSplitMaxSegs);  // [S]
-            uint64_t* digit = lds64 + 2 * kRowPart + kSplitMaxSegs + kSplitMaxSegs / 2;  // [256] masses by the next 8 bits
-            int32_t* few = reinterpret_cast<int32_t*>(digit + 256);                       // positions of the crossing digit's entries
-            __syncthreads();
-            if (g.wv == 0) before[g.lane] = wave_incl_sum(n_l) - n_l;
-            if (g.t == 0) s.n = 0;
-            digit[g.t] = 0;
-            __syncthreads();
-            if (g.t < S) kept_s[g.t] = get(segs[g.t].kept);
-#pragma unroll 1
-            for (uint32_t p = g.t; p < n; p += kTW) {  // (a few hundred entries at most: one round, mostly)
-                const int sg = segment_at(before, p);
-                const uint64_t k = get(segs[sg].part[p - before[sg]]);
-                const float m = mass_of(exp_neg(key2f((uint32_t)(k >> 32))), Cb);
-                list[p] = k;
-                mass[p] = units(m);
-                atomicAdd((unsigned long long*)&digit[(__float_as_uint(m) >> 6) & 255u], (unsigned long long)units(m));
-            }
-            __syncthreads();
-            // the digit that holds the crossing, then its entries (a few) compared with each other
-            double digit_below, digit_total;
-            const uint32_t dc = (uint32_t)crossing(digit[g.t], T - below, digit_below, digit_total);
-#pragma unroll 1
-            for (uint32_t p = g.t; p < n; p += kTW)
-                if (((__float_as_uint(mass_of(exp_neg(key2f((uint32_t)(list[p] >> 32))), Cb)) >> 6) & 255u) == dc)
-                    few[atomicAdd(&s.n, 1)] = (int32_t)p;
-            __syncthreads();
-            const int m = s.n;
-            const uint64_t rest = (uint64_t)(T - below - digit_below);
-            for (int j = g.t; j < m; j += kTW) {
-                const int pj = few[j];
-                const uint64_t k = list[pj];
-                uint64_t lower = 0;
-                for (int i = 0; i < m; i++) lower += list[few[i]] < k ? mass[few[i]] : 0ull;
-                if (lower <= rest && rest - lower < mass[pj]) s.slot[3][0] = k;  // exactly one entry
-            }
-            __syncthreads();
-            const uint64_t cut = s.slot[3][0];
-#pragma unroll 1
-            for (uint32_t p = g.t; p < n; p += kTW)
-                if (list[p] >= cut)
-                    atomicAdd((unsigned long long*)&kept_s[(uint32_t)list[p] / (uint32_t)L], (unsigned long long)mass[p]);
-            __syncthreads();
-            kept_l = in ? (double)kept_s[g.lane] : 0.0;
-            ckey = (uint32_t)(cut >> 32);
-            cidx = (uint32_t)cut;
-        }
-    } else {
-        double ls = 0.0;
-#pragma unroll
-        for (int e = 0; e < NE; e++) {
-            if (e % 4 == 0) __builtin_amdgcn_sched_barrier(0);
-            ls += (double)units(v[e]);
-        }
-        ls = g.dsum(ls);
-        if (g.t == 0) put(me.kept, (uint64_t)ls);
-        if (!meet(&row.meet[1], S, g, s)) return kEndUnsampled;
-        kept_l = in ? (double)get(segs[g.lane].kept) : 0.0;
-    }
-
-    // ---- draw: the first kept entry whose inclusive prefix mass exceeds floor(u * kept mass)
-    const double incl = wave_incl_sum(kept_l);
-    const double D = floor(u * readlane_d(incl, 63));
-    const uint64_t holds = __ballot(D >= incl - kept_l && D - (incl - kept_l) < kept_l);
-    if (!holds) return kEndUnsampled;  // no crossing (u at or above 1, NaN)
-    if ((int)__builtin_ctzll(holds) != seg) return kEndLeave;
-    const double rest = D - readlane_d(incl - kept_l, seg);
-    if (topp) {
-        // a bit per entry of the segment: those that go if they are of the cut's part (with ties the ones
-        // before the cut index, else this segment's list decides)
+    double kept_l = 0.0;      // lane l: the kept mass of segment l
+    // The entries that go, by a bit each in LDS: those of the cut's part that are below (ckey, cidx) (with
+    // ties the ones before the cut index, else this segment's list decides).
+    auto drop = [&]() {
         uint32_t* gone = reinterpret_cast<uint32_t*>(lds64);
         __syncthreads();
         for (int w = g.t; w < L / 32; w += kTW) {
@@ -760,13 +563,261 @@ __device__ __forceinline__ SplitEnd split_row(const SampleArgs& a, int vec, int 
             const uint32_t nib = gone[32 * c + (g.t >> 3)] >> (4 * (g.t & 7));
 #pragma unroll
             for (int j = 0; j < 4; j++) {
-                const uint32_t q = __float_as_uint(v[4 * c + j]) >> 14;
+                const uint32_t q = part_of(v[4 * c + j]);
                 const uint32_t first_kept = qcut + ((nib >> j) & 1u);
                 v[4 * c + j] = q < first_kept ? 0.0f : v[4 * c + j];
             }
             __builtin_amdgcn_sched_barrier(0);
         }
+        __syncthreads();
+    };
+    // Stage 0 (top-k above kKMax): weights 1, the cut at the k-th largest value, ties kept; entries of mass
+    // zero count as below it (they have no part in any sum). Stage 1: the top-p cut, weights the masses.
+    auto locate = [&](auto which) -> bool {
+        constexpr int stage = decltype(which)::value;
+        uint32_t* meets = &row.meet[1 + 3 * stage];
+        auto weight = [&](float q) -> uint64_t { return stage ? units(q) : 1ull; };
+#pragma unroll
+        for (int e = 0; e < NE; e++) {
+            if (e % 4 == 0) __builtin_amdgcn_sched_barrier(0);
+            const uint32_t b = __float_as_uint(v[e]);
+            if (b) atomicAdd((unsigned long long*)&lds64[(b >> 17) - base17], (unsigned long long)weight(v[e]));
+        }
+        __syncthreads();
+        uint64_t own = 0;  // thread t: this segment's mass in bucket t
+        if (g.t < kCoarse) {
+#pragma unroll
+            for (int i = 0; i < 16; i++) own += lds64[16 * g.t + ((i + g.t) & 15)];
+            if (own) sum_up(row.coarse[stage][g.t], own);
+        }
+        if (!meet(&meets[0], S, g, s)) return false;
+        // the bucket where the ascending cumulative mass crosses T
+        auto crossing = [&](uint64_t h, double rest, double& below, double& total) -> int {
+            const double run = g.excl((double)h, total);
+            // (rest negative: T itself is sought)
+            const double t0 = rest >= 0.0 ? rest : stage ? floor(thr * total) : total - (double)K;
+            if (h != 0 && run <= t0 && t0 - run < (double)h) {
+                s.wcand[0] = g.t;
+                s.slot[2][0] = (uint64_t)__double_as_longlong(run);
+            }
+            __syncthreads();
+            total = readlane_d(total, 0);  // (uniform: in scalar registers from here)
+            below = readlane_d(__longlong_as_double((long long)s.slot[2][0]), 0);
+            return __builtin_amdgcn_readfirstlane(s.wcand[0]);
+        };
+        uint64_t h = g.t < kCoarse ? get(row.coarse[stage][g.t]) : 0ull;
+        double below, total;
+        const int bc = crossing(h, -1.0, below, total);
+        const double T = stage ? floor(thr * total) : total - (double)K;
+        if (T >= total) return false;  // top-p so small that only the last entry stays
+        if (T < 0.0) {                         // at most K entries have mass: all of them stay
+            __syncthreads();
+            for (int i = g.t; i < kFineMass; i += kTW) lds64[i] = 0;
+            __syncthreads();
+            return true;
+        }
+        double kept = readlane_d(g.dsum(g.t > bc ? (double)own : 0.0), 0);  // this segment's mass above the bucket
+        // its 128 parts
+        if (g.t < kSub) lds64[g.t] = 0;
+        __syncthreads();
+        const uint32_t q21 = (uint32_t)bc + (base17 >> 4);
+#pragma unroll
+        for (int e = 0; e < NE; e++) {
+            if (e % 4 == 0) __builtin_amdgcn_sched_barrier(0);
+            const uint32_t b = __float_as_uint(v[e]);
+            if ((b >> 21) == q21) atomicAdd((unsigned long long*)&lds64[(b >> 14) & (kSub - 1)], (unsigned long long)weight(v[e]));
+        }
+        __syncthreads();
+        own = g.t < kSub ? lds64[g.t] : 0;
+        if (own) sum_up(row.sub[stage][g.t], own);
+        if (!meet(&meets[1], S, g, s)) return false;
+        h = g.t < kSub ? get(row.sub[stage][g.t]) : 0ull;
+        double sub_below, sub_total;
+        const int bf = crossing(h, T - below, sub_below, sub_total);
+        below += sub_below;
+        qcut = (q21 << 7) + (uint32_t)bf;
+        kept += readlane_d(g.dsum(g.t > bf ? (double)own : 0.0), 0);
+        // the part's entries as (d, index) keys (stage 0: by value): their indices first, then their values
+        // read again, all at once (few: one each per thread)
+        auto key_of = [&](int i) -> uint32_t {
+            const float x = X(i, xrow[i]);
+            return f2key(stage ? x - mx : x);
+        };
+        auto mass_of_key = [&](uint32_t key) -> float { return mass_of(exp_neg(stage ? key2f(key) : key2f(key) - mx), Cb); };
+        if (g.t == 0) s.n = 0;
+        int32_t* mine = reinterpret_cast<int32_t*>(lds64 + kSub);  // indices of this segment's entries of the part
+        __syncthreads();
+#pragma unroll
+        for (int c = 0; c < NC; c++) {
+            bool is[4];
+            int n4 = 0;
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                is[j] = part_of(v[4 * c + j]) == qcut;
+                n4 += is[j] ? 1 : 0;
+            }
+            if (n4) {
+                int at = atomicAdd(&s.n, n4);
+#pragma unroll
+                for (int j = 0; j < 4; j++)
+                    if (is[j]) mine[at++ & (kMine - 1)] = lo + 1024 * c + 4 * g.t + j;
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        __syncthreads();
+        uint32_t kmin = 0xffffffffu, kmax = 0;
+        own_n = __builtin_amdgcn_readfirstlane(s.n);
+        if (own_n <= kMine) {
+            for (int j = g.t; j < own_n; j += kTW) {
+                const int i = mine[j];
+                const uint32_t key = key_of(i);
+                kmin = min(kmin, key);
+                kmax = max(kmax, key);
+                if (j < kSegPart) put(me.part[j], ((uint64_t)key << 32) | (uint32_t)i);
+            }
+        } else {  // many: ties, most likely; each thread reads its own
+#pragma unroll 4
+            for (int e = 0; e < NE; e++) {
+                const int i = lo + 1024 * (e / 4) + 4 * g.t + (e & 3);
+                bool in_part = false;
+#pragma unroll
+                for (int q = 0; q < NE; q++) in_part |= q == e && part_of(v[q]) == qcut;
+                const uint32_t key = in_part ? key_of(i) : 0u;
+                kmin = in_part ? min(kmin, key) : kmin;
+                kmax = max(kmax, key);
+            }
+        }
+        kmin = g.umin(kmin);
+        kmax = g.umax(kmax);
+        if (g.t == 0) {
+            put(me.n, (uint32_t)own_n);
+            put(me.kmin, kmin);
+            put(me.kmax, kmax);
+            put(me.kept, (uint64_t)kept);
+        }
+        if (!meet(&meets[2], S, g, s)) return false;
+        const uint32_t n_l = in ? get(segs[g.lane].n) : 0u;
+        const uint32_t n = wave_sum(n_l);
+        kept_l = in ? (double)get(segs[g.lane].kept) : 0.0;
+        kmin = wave_umin(in ? get(segs[g.lane].kmin) : 0xffffffffu);
+        kmax = wave_umax(in ? get(segs[g.lane].kmax) : 0u);
+        tied = kmin == kmax;
+        if (tied) {
+            // one key (ties, or one entry): the crossing follows index order among them
+            const double w = (double)weight(mass_of_key(kmin));
+            const uint32_t nth = (uint32_t)((T - below) / w);  // entries of the part that go (exact integers)
+            const uint32_t before = wave_incl_sum(n_l) - n_l;
+            const uint32_t go_l = min(n_l, nth > before ? nth - before : 0u);
+            kept_l += w * (double)(n_l - go_l);
+            ckey = kmin;
+            const uint32_t go = readlane(go_l, seg);  // this segment's first `go` tied entries in index order go
+            cidx = 0;
+            if (!stage) {
+                // (ties at the k-th largest are kept)
+            } else if (go == (uint32_t)own_n) {
+                cidx = 0x7fffffffu;
+            } else if (go) {  // uniform: the index of entry number `go` among them
+                uint32_t run = 0;
+#pragma unroll 1
+                for (int c = 0; c < NC; c++) {
+                    uint32_t m4 = 0;
+#pragma unroll
+                    for (int e = 0; e < NE; e++)
+                        if (e / 4 == c) m4 |= part_of(v[e]) == qcut ? 1u << (e & 3) : 0u;
+                    uint32_t t4;
+                    const uint32_t ex = run + g.excl((uint32_t)__builtin_popcount(m4), t4);
+                    if (go >= ex && go < ex + (uint32_t)__builtin_popcount(m4)) {
+                        for (uint32_t k = go - ex; k; k--) m4 &= m4 - 1;
+                        s.wcand[1] = lo + 1024 * c + 4 * g.t + __builtin_ctz(m4);
+                    }
+                    run += t4;
+                }
+                __syncthreads();
+                cidx = (uint32_t)s.wcand[1];
+            }
+        } else if (n > (uint32_t)kRowPart || __ballot(n_l > (uint32_t)kSegPart)) {
+            return false;
+        } else {
+            uint64_t* list = lds64;                   // [n] keys
+            uint64_t* mass = lds64 + kRowPart;        // [n] their masses
+            uint64_t* kept_s = lds64 + 2 * kRowPart;  // [S]
+            uint32_t* before = reinterpret_cast<uint32_t*>(kept_s + kSplitMaxSegs);  // [S]
+            uint64_t* digit = lds64 + 2 * kRowPart + kSplitMaxSegs + kSplitMaxSegs / 2;  // [256] masses by the next 8 bits
+            int32_t* few = reinterpret_cast<int32_t*>(digit + 256);                       // positions of the crossing digit's entries
+            __syncthreads();
+            if (g.wv == 0) before[g.lane] = wave_incl_sum(n_l) - n_l;
+            if (g.t == 0) s.n = 0;
+            digit[g.t] = 0;
+            __syncthreads();
+            if (g.t < S) kept_s[g.t] = get(segs[g.t].kept);
+#pragma unroll 1
+            for (uint32_t p = g.t; p < n; p += kTW) {  // (a few hundred entries at most: one round, mostly)
+                const int sg = segment_at(before, p);
+                const uint64_t k = get(segs[sg].part[p - before[sg]]);
+                const float m = mass_of_key((uint32_t)(k >> 32));
+                list[p] = k;
+                mass[p] = weight(m);
+                atomicAdd((unsigned long long*)&digit[(__float_as_uint(m) >> 6) & 255u], (unsigned long long)weight(m));
+            }
+            __syncthreads();
+            // the digit that holds the crossing, then its entries (a few) compared with each other
+            double digit_below, digit_total;
+            const uint32_t dc = (uint32_t)crossing(digit[g.t], T - below, digit_below, digit_total);
+#pragma unroll 1
+            for (uint32_t p = g.t; p < n; p += kTW)
+                if (((__float_as_uint(mass_of_key((uint32_t)(list[p] >> 32))) >> 6) & 255u) == dc)
+                    few[atomicAdd(&s.n, 1)] = (int32_t)p;
+            __syncthreads();
+            const int m = s.n;
+            const uint64_t rest = (uint64_t)(T - below - digit_below);
+            for (int j = g.t; j < m; j += kTW) {
+                const int pj = few[j];
+                const uint64_t k = list[pj];
+                uint64_t lower = 0;
+                for (int i = 0; i < m; i++) lower += list[few[i]] < k ? mass[few[i]] : 0ull;
+                if (lower <= rest && rest - lower < mass[pj]) s.slot[3][0] = k;  // exactly one entry
+            }
+            __syncthreads();
+            const uint64_t cut = s.slot[3][0];
+#pragma unroll 1
+            for (uint32_t p = g.t; p < n; p += kTW)
+                if (list[p] >= cut)
+                    atomicAdd((unsigned long long*)&kept_s[(uint32_t)list[p] / (uint32_t)L], (unsigned long long)mass[p]);
+            __syncthreads();
+            kept_l = in ? (double)kept_s[g.lane] : 0.0;
+            ckey = (uint32_t)(cut >> 32);
+            cidx = stage ? (uint32_t)cut : 0u;
+        }
+        if (!stage) {
+            drop();
+            for (int i = g.t; i < kFineMass; i += kTW) lds64[i] = 0;  // stage 1's histogram
+            __syncthreads();
+        }
+        return true;
+    };
+    if (count_first && !locate(std::integral_constant<int, 0>())) return kEndUnsampled;
+    if (topp && !locate(std::integral_constant<int, 1>())) return kEndUnsampled;
+    if (!topp) {
+        double ls = 0.0;
+#pragma unroll
+        for (int e = 0; e < NE; e++) {
+            if (e % 4 == 0) __builtin_amdgcn_sched_barrier(0);
+            ls += (double)units(v[e]);
+        }
+        ls = g.dsum(ls);
+        if (g.t == 0) put(me.kept, (uint64_t)ls);
+        if (!meet(&row.meet[7], S, g, s)) return kEndUnsampled;
+        kept_l = in ? (double)get(segs[g.lane].kept) : 0.0;
     }
+
+    // ---- draw: the first kept entry whose inclusive prefix mass exceeds floor(u * kept mass)
+    const double incl = wave_incl_sum(kept_l);
+    const double D = floor(u * readlane_d(incl, 63));
+    const uint64_t holds = __ballot(D >= incl - kept_l && D - (incl - kept_l) < kept_l);
+    if (!holds) return kEndUnsampled;  // no crossing (u at or above 1, NaN)
+    if ((int)__builtin_ctzll(holds) != seg) return kEndLeave;
+    const double rest = D - readlane_d(incl - kept_l, seg);
+    if (topp) drop();
     double* sweep = reinterpret_cast<double*>(lds64);  // [NC][waves]
     __syncthreads();
 #pragma unroll
@@ -821,9 +872,9 @@ __global__ __launch_bounds__(kTW) __attribute__((amdgpu_waves_per_eu(4))) void s
     if (end != kEndGeneral) {
         if (!arrive_last(&row.left, S, g, s)) return;
         // clear the row for the next call
-        if (g.t < kCoarse) put(row.coarse[g.t], uint64_t(0));
-        if (g.t < kSub) put(row.sub[g.t], uint64_t(0));
-        if (g.t < 4) put(row.meet[g.t], 0u);
+        for (int i = g.t; i < 2 * kCoarse; i += kTW) put(row.coarse[0][i], uint64_t(0));
+        for (int i = g.t; i < 2 * kSub; i += kTW) put(row.sub[0][i], uint64_t(0));
+        if (g.t < 8) put(row.meet[g.t], 0u);
         if (g.t == 0) put(row.left, 0u);
         if (end == kEndLeave) return;
     }
