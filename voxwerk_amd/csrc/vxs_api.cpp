@@ -114,7 +114,6 @@ struct vxs_history {
     int32_t* ids = nullptr;  // [slots][cap]
     int32_t* len = nullptr;  // [slots]
     int32_t* rng = nullptr;  // [slots][2][kRngWords]: talker and code-predictor generators
-    vxs::StoreDesc* desc = nullptr;  // the three pointers and the shape, in device memory
     std::vector<uint8_t> seeded;  // host record of vxs_history_seed per slot
 };
 
@@ -307,7 +306,7 @@ void set_resident(vxs::SampleArgs& a, const vxs_history* h, const int32_t* d_slo
     a.hist_len = h->len;
     a.hist_cap = h->cap;
     a.hist_slots = h->slots;
-    a.store = h->desc;
+    a.store_rng = h->rng;
     if (append) a.kflags |= vxs::KF_APPEND;
     if (rng_stream >= 0) a.kflags |= vxs::KF_RNG | (rng_stream == 1 ? vxs::KF_RNG_SUB : 0u);
 }
@@ -940,12 +939,6 @@ VXS_API int vxs_history_create(vxs_ctx* ctx, int slots, int cap, vxs_history** o
         if (e == hipSuccess) e = hipMalloc(&h->rng, rng_bytes);
         if (e == hipSuccess) e = hipMemsetAsync(h->len, 0, sizeof(int32_t) * (size_t)slots, ctx->stream);
         if (e == hipSuccess) e = hipMemsetAsync(h->rng, 0, rng_bytes, ctx->stream);
-        if (e == hipSuccess) e = hipMalloc(&h->desc, sizeof(vxs::StoreDesc));
-        if (e == hipSuccess) {
-            const vxs::StoreDesc d{h->ids, h->len, h->rng, cap, slots};
-            e = hipMemcpyAsync(h->desc, &d, sizeof d, hipMemcpyHostToDevice, ctx->stream);
-            if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
-        }
         if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
         if (e != hipSuccess) {
             vxs_history_destroy(h);
@@ -965,7 +958,6 @@ VXS_API void vxs_history_destroy(vxs_history* h) {
     if (h->ids) (void)hipFree(h->ids);
     if (h->len) (void)hipFree(h->len);
     if (h->rng) (void)hipFree(h->rng);
-    if (h->desc) (void)hipFree(h->desc);
     delete h;
 }
 

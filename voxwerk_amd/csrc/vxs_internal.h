@@ -18,16 +18,6 @@ enum : uint32_t {
     KF_RNG_SUB = 8u,             //   the code predictor's (else the talker's)
 };
 
-// A resident store as the kernels see it (vxs_history, one copy in device memory per store):
-// ids [slots][cap], lengths [slots], generators [slots][2][kRngWords].
-struct StoreDesc {
-    int32_t* ids;
-    int32_t* len;
-    int32_t* rng;
-    int cap;
-    int slots;
-};
-
 struct SampleArgs {
     int rows;
     int vocab;
@@ -42,11 +32,11 @@ struct SampleArgs {
     const int32_t* hist_len;
     int hist_cap;
     int hist_slots;
-    // With a resident store (`store`, in device memory), the row's step ends in the kernel
-    // (put_id): with KF_APPEND the slot takes the sampled id, and with KF_RNG a sampled row's
-    // uniform is the next NextDouble() of generator 2 * slot + (KF_RNG_SUB ? 1 : 0) instead of u[r]
-    // (read by row_uniform, advanced once by put_id).
-    const struct StoreDesc* store;
+    // With a resident store (its generators, [slots][2][kRngWords], set) the row's step ends in the
+    // kernel (put_id): with KF_APPEND the slot takes the sampled id (hist_ids and hist_len are the
+    // store's own arrays), and with KF_RNG a sampled row's uniform is the next NextDouble() of generator
+    // 2 * slot + (KF_RNG_SUB ? 1 : 0) instead of u[r], advanced once by put_id.
+    int32_t* store_rng;
     const vxs_params* params;
     int params_stride;
     const double* u;
@@ -125,16 +115,19 @@ struct RngStep {
     int32_t v;
     int i, j;
 };
-__device__ __forceinline__ RngStep rng_peek(const int32_t* st) {
+__device__ __forceinline__ int32_t rng_value(int32_t wi, int32_t wj) {
     constexpr int32_t kMbig = 0x7FFFFFFF;
+    int32_t v = (int32_t)((uint32_t)wi - (uint32_t)wj);
+    if (v == kMbig) v--;
+    if (v < 0) v = (int32_t)((uint32_t)v + (uint32_t)kMbig);
+    return v;
+}
+__device__ __forceinline__ RngStep rng_peek(const int32_t* st) {
     int i = st[56] + 1;
     if (i >= 56) i = 1;
     int j = st[57] + 1;
     if (j >= 56) j = 1;
-    int32_t v = (int32_t)((uint32_t)st[i] - (uint32_t)st[j]);
-    if (v == kMbig) v--;
-    if (v < 0) v = (int32_t)((uint32_t)v + (uint32_t)kMbig);
-    return {v, i, j};
+    return {rng_value(st[i], st[j]), i, j};
 }
 __device__ __forceinline__ void rng_commit(int32_t* st, const RngStep& t) {
     st[t.i] = t.v;
@@ -144,47 +137,84 @@ __device__ __forceinline__ void rng_commit(int32_t* st, const RngStep& t) {
 // NextDouble() = InternalSample() * (1.0 / int.MaxValue) (Sampler.cs:77).
 __device__ __forceinline__ double rng_double(int32_t v) { return (double)v * (1.0 / 2147483647.0); }
 
+// Row r's generator state, or null for a slot outside the store.
+__device__ __forceinline__ int32_t* row_rng(const SampleArgs& a, int r) {
+    const int s = a.hist_slot[r];
+    if ((unsigned)s >= (unsigned)a.hist_slots) return nullptr;
+    return a.store_rng + ((int64_t)s * 2 + ((a.kflags & KF_RNG_SUB) ? 1 : 0)) * kRngWords;
+}
+
 // The uniform row r's draw uses: u[r], or with a resident store's generators the next NextDouble()
 // of its slot's generator, read without advancing it (put_id advances it once for the row). Any
 // number of threads may call it before the row's put_id. 0 for a slot outside the store.
-__device__ __forceinline__ int32_t* slot_rng(const SampleArgs& a, const StoreDesc& d, int s) {
-    return d.rng + ((int64_t)s * 2 + ((a.kflags & KF_RNG_SUB) ? 1 : 0)) * kRngWords;
-}
 __device__ __forceinline__ double row_uniform(const SampleArgs& a, int r) {
     if (a.kflags & KF_RNG) {
-        const StoreDesc d = *a.store;
-        const int s = a.hist_slot[r];
-        if ((unsigned)s >= (unsigned)d.slots) return 0.0;
-        return rng_double(rng_peek(slot_rng(a, d, s)).v);
+        const int32_t* st = row_rng(a, r);
+        return st ? rng_double(rng_peek(st).v) : 0.0;
     }
     if (a.row_direct) return a.direct_u;
     return a.u ? a.u[r] : 0.0;
 }
 
+// row_uniform in three parts, for a row whose time is a chain of latencies: a generator's draw is two
+// dependent reads after its slot (the table positions, the words there) and u[r] one, each begun while
+// the row works on something else and none waited for at the draw.
+struct UniformAhead {
+    int32_t* st;        // the row's generator, or null
+    int i, j;           // its positions as stored
+    int32_t wi, wj;     // the words there after the step
+    double u;
+    __device__ __forceinline__ void begin(const SampleArgs& a, int r) {
+        st = (a.kflags & KF_RNG) ? row_rng(a, r) : nullptr;
+        i = j = 0;
+        u = 0.0;
+        if (st) {
+            i = st[56];
+            j = st[57];
+        }
+    }
+    __device__ __forceinline__ void words(const SampleArgs& a, int r) {
+        wi = wj = 0;
+        if (!st) {
+            if (!(a.kflags & KF_RNG)) u = a.row_direct ? a.direct_u : a.u ? a.u[r] : 0.0;
+            return;
+        }
+        i = i + 1 >= 56 ? 1 : i + 1;
+        j = j + 1 >= 56 ? 1 : j + 1;
+        wi = st[i];
+        wj = st[j];
+    }
+    __device__ __forceinline__ RngStep step() const { return {rng_value(wi, wj), i, j}; }
+    __device__ __forceinline__ double value() const { return st ? rng_double(step().v) : u; }
+};
+
 // The one store of row r's result, by one thread after every thread of the row has taken its
 // uniform. With a resident store it also ends the row's step (the order of the batched
 // generator's loop, TalkerGenerator.cs:369-374): a row whose slot lies outside the store fails with
 // VXS_ERR_INVALID_ARG; a sampled row advances its slot's generator (one NextDouble per sampled
-// Select, whatever the outcome, Sampler.cs:77); with `append` a sampled id joins the slot's
-// history (History.Add), or the row fails with VXS_ERR_HISTORY_FULL when the slot is full.
-__device__ __forceinline__ void put_id(const SampleArgs& a, int r, int id) {
-    if (a.store) {  // the descriptor is read here, at the row's end
-        const StoreDesc d = *a.store;
+// Select, whatever the outcome, Sampler.cs:77; `ahead` when its step was read ahead); with KF_APPEND a
+// sampled id joins the slot's history (History.Add), or the row fails with VXS_ERR_HISTORY_FULL when the
+// slot is full.
+__device__ __forceinline__ void put_id(const SampleArgs& a, int r, int id, const UniformAhead* ahead = nullptr) {
+    if (a.store_rng) {
         const int s = a.hist_slot[r];
-        if ((unsigned)s >= (unsigned)d.slots) {
+        if ((unsigned)s >= (unsigned)a.hist_slots) {
             id = VXS_ERR_INVALID_ARG;
         } else {
-            if ((a.kflags & KF_RNG) && a.params[(int64_t)r * a.params_stride].do_sample) {
-                int32_t* st = slot_rng(a, d, s);
+            if (ahead && ahead->st) {  // (the draw of a sampled row)
+                rng_commit(ahead->st, ahead->step());
+            } else if ((a.kflags & KF_RNG) && a.params[(int64_t)r * a.params_stride].do_sample) {
+                int32_t* st = row_rng(a, r);
                 rng_commit(st, rng_peek(st));
             }
             if ((a.kflags & KF_APPEND) && id >= 0) {
-                const int n = d.len[s];
-                if ((unsigned)n >= (unsigned)d.cap) {
+                int32_t* len = const_cast<int32_t*>(a.hist_len) + s;
+                const int n = *len;
+                if ((unsigned)n >= (unsigned)a.hist_cap) {
                     id = VXS_ERR_HISTORY_FULL;
                 } else {
-                    d.ids[(int64_t)s * d.cap + n] = id;
-                    d.len[s] = n + 1;
+                    const_cast<int32_t*>(a.hist_ids)[(int64_t)s * a.hist_cap + n] = id;
+                    *len = n + 1;
                 }
             }
         }

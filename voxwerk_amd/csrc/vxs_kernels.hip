@@ -505,7 +505,8 @@ template <int NC>
 constexpr int kWavesPerEu = NC <= 3 ? 4 : 1;
 
 // One row by the whole 256-thread workgroup (every thread calls it; it returns uniformly).
-template <int NC>
+// kAhead: the draw's uniform is read in parts along the way (launch_nc has the rule); else at the draw.
+template <int NC, bool kAhead>
 __device__ __forceinline__ void row_block(const SampleArgs& a, int vec, int r, RowSmem<NC>& sm) {
     using C = Cfg<NC>;
     constexpr int NE = C::NE;
@@ -548,6 +549,8 @@ __device__ __forceinline__ void row_block(const SampleArgs& a, int vec, int r, R
         P = a.params[(int64_t)r * a.params_stride];
     HistRange hr{0, 0};
     if (has_history(a)) hr = history_range(a, r);
+    UniformAhead un;  // the draw's uniform, read in parts along the way
+    if constexpr (kAhead) un.begin(a, r);
     const bool pen_on = P.rep_penalty != 1.0f && has_history(a);
     constexpr int HP = 8;  // ids per thread fetched up front (2048 per row), in flight with the row
     const int h0 = hr.h0, h1 = pen_on ? hr.h1 : hr.h0;
@@ -708,6 +711,8 @@ __device__ __forceinline__ void row_block(const SampleArgs& a, int vec, int r, R
                 if (eidx(e) < V) prow[eidx(e)] = 0.0;
         return;
     }
+
+    if constexpr (kAhead) un.words(a, r);
 
     // ---- S4: temperature, and the finite-input contract
     const float invT = P.temperature == 1.0f ? 1.0f : 1.0f / P.temperature;
@@ -911,7 +916,8 @@ __device__ __forceinline__ void row_block(const SampleArgs& a, int vec, int r, R
     write_logits();
 
     const float m = mx;
-    const double u = row_uniform(a, r);
+    const double u = kAhead ? un.value() : row_uniform(a, r);
+    const UniformAhead* const ahead = kAhead ? &un : nullptr;
 
     if (cnt <= (uint32_t)kCandMax) {
         // ================= exact regime: the reference's sequential fp64 arithmetic =================
@@ -999,7 +1005,7 @@ __device__ __forceinline__ void row_block(const SampleArgs& a, int vec, int r, R
                 const int nl = (int)cnt;
                 const float xl = g.lane < nl ? cx[g.lane] : 0.0f;
                 const int pick = wave_exact(xl, ci, nl, m, topp, P.top_p, u, ex.ps, prow, g.lane);
-                if (g.lane == 0) put_id(a, r, pick);
+                if (g.lane == 0) put_id(a, r, pick, ahead);
             }
             return;
         }
@@ -1060,7 +1066,7 @@ __device__ __forceinline__ void row_block(const SampleArgs& a, int vec, int r, R
         }
         if (g.wv == 0) {  // inverse-CDF draw in index order                              :77-87
             const int pick = wave_draw(ex.cp, ex.ci, n, u);
-            if (g.lane == 0) put_id(a, r, pick);
+            if (g.lane == 0) put_id(a, r, pick, ahead);
         }
         if (prow)
             for (int j = g.t; j < n; j += kT) prow[ex.ci[j]] = ex.cp[j];
@@ -1362,7 +1368,7 @@ __device__ __forceinline__ void row_block(const SampleArgs& a, int vec, int r, R
         pick = g.imax(li, kSiteLast);
         if (pick < 0) pick = 0;
     }
-    if (g.t == 0) put_id(a, r, pick);
+    if (g.t == 0) put_id(a, r, pick, ahead);
     if (prow) {
         double se = 0.0;
 #pragma unroll
@@ -1389,11 +1395,11 @@ __device__ __forceinline__ void signal_done(const SampleArgs& a) {
     }
 }
 
-template <int NC>
+template <int NC, bool kAhead>
 __global__ __launch_bounds__(kT) __attribute__((amdgpu_waves_per_eu(kWavesPerEu<NC>))) void sample_rows_kernel(
     SampleArgs a, int vec) {
     __shared__ RowSmem<NC> sm;
-    row_block<NC>(a, vec, blockIdx.x, sm);
+    row_block<NC, kAhead>(a, vec, blockIdx.x, sm);
     if (a.done_flag) signal_done(a);
 }
 
@@ -1436,18 +1442,28 @@ __global__ __launch_bounds__(kT) __attribute__((amdgpu_waves_per_eu(4))) void sa
     static_assert(kWaves == 4, "four rows per workgroup");
     if constexpr (kPrio)
         if (b0 | b1 | b2 | b3) __builtin_amdgcn_s_setprio(3);  // the slowest rows: all four waves alike
-    if (b0) row_block<NC>(a, vec, r0, sm.row);
+    if (b0) row_block<NC, false>(a, vec, r0, sm.row);
     if (b0 && (b1 | b2 | b3)) __syncthreads();  // LDS is reused by the next row
-    if (b1) row_block<NC>(a, vec, r0 + 1, sm.row);
+    if (b1) row_block<NC, false>(a, vec, r0 + 1, sm.row);
     if (b1 && (b2 | b3)) __syncthreads();
-    if (b2) row_block<NC>(a, vec, r0 + 2, sm.row);
+    if (b2) row_block<NC, false>(a, vec, r0 + 2, sm.row);
     if (b2 && b3) __syncthreads();
-    if (b3) row_block<NC>(a, vec, r0 + 3, sm.row);
+    if (b3) row_block<NC, false>(a, vec, r0 + 3, sm.row);
 }
 
 template <int NC>
 hipError_t launch_nc(const SampleArgs& a, int vec, hipStream_t stream) {
-    hipLaunchKernelGGL((sample_rows_kernel<NC>), dim3(a.rows), dim3(kT), 0, stream, a, vec);
+    // The uniform read ahead for rows that draw from a resident store's generator and for polled host
+    // calls (24-sequence device step 207 -> 195 us, frame of 15 host calls 343 -> 334); for uniforms in
+    // device memory it costs more than the one late read (256 x 3072: 11.46 us, 11.26 without).
+    // Vocabularies above 3072 are neither talker's nor code predictor's and have the one instance.
+    if constexpr (NC <= 3) {
+        if ((a.kflags & KF_RNG) || a.done_flag) {
+            hipLaunchKernelGGL((sample_rows_kernel<NC, true>), dim3(a.rows), dim3(kT), 0, stream, a, vec);
+            return hipGetLastError();
+        }
+    }
+    hipLaunchKernelGGL((sample_rows_kernel<NC, false>), dim3(a.rows), dim3(kT), 0, stream, a, vec);
     return hipGetLastError();
 }
 

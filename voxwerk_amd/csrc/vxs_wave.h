@@ -144,7 +144,7 @@ template <int NS>
 __device__ __forceinline__ int wave_prepare(const SampleArgs& a, int r, int lane, const vxs_params& P, WaveRow<NS>& w) {
     using namespace wave;
     // outputs, the penalty alone and resident stores (whose step ends in put_id) take the general path
-    if (a.out_logits || a.out_probs || (a.kflags & KF_STOP_AFTER_PENALTY) || a.store) return 1;
+    if (a.out_logits || a.out_probs || (a.kflags & KF_STOP_AFTER_PENALTY) || a.store_rng) return 1;
     if (P.do_sample && P.top_k > kL && P.top_k < a.vocab) return 1;  // top-k beyond one wave's candidates
     const bool pen_on = P.rep_penalty != 1.0f && has_history(a);
     HistRange hr{0, 0};
