@@ -975,6 +975,13 @@ __device__ __forceinline__ bool ordered_tail(const SampleArgs& a, int vec, int r
     __syncthreads();
 
     __builtin_amdgcn_s_setprio(0);
+    if (n <= 64 && !prow) {  // one candidate per lane of the worker wave
+        if (!worker) return false;
+        const int pick = wave_exact(g.lane < n ? s.ex.cx[g.lane] : 0.0f, s.ex.ci, n, mx, P.top_p < 1.0f, P.top_p, row_uniform(a, r),
+                                    reinterpret_cast<double*>(&s.widx[0][0]), nullptr, g.lane);
+        if (g.lane == 0) put_id(a, r, pick);
+        return false;
+    }
     // ---- all waves: thread t holds candidate t (index order); its position in (d, index) order,
     // counted over the keys eight at a time, and its exp(d)                        Sampler.cs:57
     if (g.t < n) {
