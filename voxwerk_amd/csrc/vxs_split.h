@@ -149,7 +149,7 @@ __device__ __forceinline__ int segment_at(const uint32_t* before, uint32_t p) {
 // segments each) into registers in index order, then the ordered pass's tail. True: the general algorithm
 // must sample the row (nothing written).
 __device__ __forceinline__ bool split_topk_finish(const SampleArgs& a, int vec, int r, const vxs_params& P, const RowX& X, BlkW& g,
-                                                  WideSmem& s, const SplitSeg* segs, int S, const float* __restrict__ xrow) {
+                                                  WideSmem& s, const SplitSeg* segs, int S, const float* __restrict__ xrow, double u) {
     const int K = P.top_k;
     const bool in = g.lane < S;
     const uint32_t my_n = in ? get(segs[g.lane].n) : 0u;
@@ -273,7 +273,7 @@ __device__ __forceinline__ bool split_topk_finish(const SampleArgs& a, int vec, 
         any_full = any_full || s.wbad[w] != 0;
     }
     if (any_full) return true;
-    return ordered_tail(a, vec, r, P, X, g, s, kk, ii, klo, khi, K, (uint32_t)K < cnt, g.wv == 0, nullptr, nullptr, xrow);
+    return ordered_tail(a, vec, r, P, X, g, s, kk, ii, klo, khi, K, (uint32_t)K < cnt, g.wv == 0, nullptr, nullptr, xrow, [&]() { return u; });
 }
 
 // What is left to do for a row when its workgroup's part is done.
@@ -481,7 +481,7 @@ __device__ __forceinline__ SplitEnd split_row(const SampleArgs& a, int vec, int 
         }
         if (!arrive_last(&row.meet[0], S, g, s)) return kEndGone;
         if (g.t == 0) put(row.meet[0], 0u);
-        return split_topk_finish(a, vec, r, P, X, g, s, segs, S, xrow) ? kEndGeneral : kEndGone;
+        return split_topk_finish(a, vec, r, P, X, g, s, segs, S, xrow, u) ? kEndGeneral : kEndGone;
     }
 
     // ---- nucleus. Meeting 0: the row's maximum and finite count

@@ -922,12 +922,13 @@ __device__ __forceinline__ float x_threshold(float tau, float invT) {
 // The tail of a row whose candidates the four waves hold in registers, in index order (wave ranges
 // ascending, slot lane + 64 q of a wave): kk the keys of the exact values (0: no entry), ii the indices,
 // [klo, khi] the workgroup's smallest and largest key, at most K ties aside at or above the k-th
-// largest. `worker` marks the wave that runs the sequential part. Returns true, before anything was
+// largest. `worker` marks the wave that runs the sequential part, uniform() the draw's uniform. Returns true, before anything was
 // written, when more candidates tie at the k-th largest than the exact regime holds.
+template <class U>
 __device__ __forceinline__ bool ordered_tail(const SampleArgs& a, int vec, int r, const vxs_params& P, const RowX& X, BlkW& g,
                                              WideSmem& s, const uint32_t (&kk)[kPerL], const int32_t (&ii)[kPerL],
                                              uint32_t klo, uint32_t khi, int K, bool topk_on, bool worker, float* orow,
-                                             double* prow, const float* __restrict__ xrow) {
+                                             double* prow, const float* __restrict__ xrow, U uniform) {
     const int V = a.vocab;
     // ---- all waves: the k-th largest of the buffered keys, the maximum, the candidates
     const uint32_t kthkey = topk_on ? block_kth_radix(kk, klo, khi, K, s.h.h3, g.t, g.lane) : 1u;
@@ -977,7 +978,7 @@ __device__ __forceinline__ bool ordered_tail(const SampleArgs& a, int vec, int r
     __builtin_amdgcn_s_setprio(0);
     if (n <= 64 && !prow) {  // one candidate per lane of the worker wave
         if (!worker) return false;
-        const int pick = wave_exact(g.lane < n ? s.ex.cx[g.lane] : 0.0f, s.ex.ci, n, mx, P.top_p < 1.0f, P.top_p, row_uniform(a, r),
+        const int pick = wave_exact(g.lane < n ? s.ex.cx[g.lane] : 0.0f, s.ex.ci, n, mx, P.top_p < 1.0f, P.top_p, uniform(),
                                     reinterpret_cast<double*>(&s.widx[0][0]), nullptr, g.lane);
         if (g.lane == 0) put_id(a, r, pick);
         return false;
@@ -1080,11 +1081,11 @@ __device__ __forceinline__ bool ordered_tail(const SampleArgs& a, int vec, int r
         if (prow)
             for (int j = g.lane; j < n; j += 64) cp[j] = cp[j] / s2;
         wave_sync();
-        const double u = row_uniform(a, r);
+        const double u = uniform();
         const int pick = wave_draw(kp, kid, nk, u);  // inverse-CDF draw in index order :77-87
         if (g.lane == 0) put_id(a, r, pick);
     } else {
-        const double u = row_uniform(a, r);
+        const double u = uniform();
         const int pick = wave_draw(cp, s.ex.ci, n, u);  // inverse-CDF draw in index order :77-87
         if (g.lane == 0) put_id(a, r, pick);
     }
@@ -1443,7 +1444,8 @@ __device__ __forceinline__ bool wide_ordered_row(const SampleArgs& a, int vec, i
         for (int w = 0; w < kWW; w++) nw += s.wslot[w];
         if (nw == 1) worker = s.wslot[g.wv] != 0;
     }
-    return ordered_tail(a, vec, r, P, X, g, s, kk, ii, klo, khi, K, topk_on, worker, orow, prow, xrow);
+    return ordered_tail(a, vec, r, P, X, g, s, kk, ii, klo, khi, K, topk_on, worker, orow, prow, xrow,
+                        [&]() { return row_uniform(a, r); });
 }
 
 // One workgroup per row: the ordered pass when the row's options allow it, else (or when that pass
