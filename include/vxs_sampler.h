@@ -123,7 +123,10 @@ VXS_API int vxs_sample(vxs_ctx* ctx, int rows, int vocab, const float* logits, i
  * Device-pointer sampling call; asynchronous on the context stream. Every pointer is device
  * memory (params included). Per-row errors land in out_ids as negative codes; call
  * vxs_synchronize to wait. For callers whose logits are already resident on the GPU (logit
- * heads on device) and for kernel-only timing.
+ * heads on device) and for kernel-only timing. Batches of at most 192 rows with vocab > 8192 split
+ * each row over several workgroups, in a workspace of about 29 MB that the context allocates at the
+ * first such call on a stream (its own, and up to four set with vxs_set_stream); where none is to be
+ * had, and on a stream that is being captured, the call takes one workgroup per row. Same ids.
  */
 VXS_API int vxs_sample_device(vxs_ctx* ctx, int rows, int vocab, const float* d_logits, int64_t ld,
                               const int32_t* d_hist_off, const int32_t* d_hist_ids,
