@@ -618,7 +618,10 @@ VXS_API void vxs_destroy(vxs_ctx* ctx) {
     if (!ctx) return;
     (void)hipSetDevice(ctx->device);
     if (ctx->stream) (void)hipStreamSynchronize(ctx->stream);
-    if (ctx->split_own.p) (void)hipFree(ctx->split_own.p);
+    if (ctx->split_own.p) {
+        (void)hipStreamSynchronize(ctx->own_stream);
+        (void)hipFree(ctx->split_own.p);
+    }
     for (SplitWs& w : ctx->split_ext) {
         if (w.recorded) (void)hipEventSynchronize(w.last);
         if (w.last) (void)hipEventDestroy(w.last);
