@@ -15,7 +15,7 @@
 //                          finds it in its registers.
 // What bounds it: with few rows the chain of reads, meetings (about 2 us each) and the finish, not the
 // bytes; 64 nucleus rows of 151936 entries take 45.7 us (one workgroup per row: 1361), of which the one
-// read of 39 MB is 8; 16 top-k rows 23.9 (73). Segments stay in registers so that no stage reads the
+// read of 39 MB is 8; 16 top-k rows 22.1 (76). Segments stay in registers so that no stage reads the
 // row again, which holds them to 128 registers (four workgroups per compute unit): larger segments with
 // three per unit took 47.6 to 61 us.
 //

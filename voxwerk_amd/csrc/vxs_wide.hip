@@ -1475,7 +1475,7 @@ size_t split_workspace_bytes() { return (sizeof(SplitRow) + sizeof(SplitSeg)) * 
 // for it. Segments of 4096 entries while the call then has at most 1024 of them (four workgroups per
 // compute unit, all resident), else of 10240; one workgroup per row when the call writes back, or has
 // rows enough to keep the compute units busy that way (us, split / one workgroup per row, top-k 50 or as
-// said: 1 x 151936 19.9 / 74, 16 x 151936 23.8 / 73, 64 32.8 / 78, 136 51.3 / 79, 200 x 20000 26.6 / 28.4,
+// said: 1 x 151936 19.9 / 74, 16 x 151936 22.1 / 76, 64 32.8 / 78, 136 51.3 / 79, 200 x 20000 26.6 / 28.4,
 // 300 x 20000 31.8 / 29.9, 128 x 151936 at top-k 200 70 / 86; nucleus, top-p 0.9: 4 x 151936 25.6 / 1017, 64
 // 45.7 / 1361, 128 82 / 1385, 300 x 20000 40.7 / 220; top-k 400: 16 x 151936 48 / 1386, 2 x 30000 31 / 289).
 static int split_segment(const SampleArgs& a) {
