@@ -204,28 +204,32 @@ __global__ __launch_bounds__(kHT) void head_i8_kernel(HeadArgs a) {
     }
 }
 
-// ---- matrix-core forms, for 8 or more rows ------------------------------------------------------
-// The hidden rows are fp32 and v_mfma_f32_16x16x32_bf16 multiplies bf16, so each x is split exactly
-// into three bf16 parts, x = h + m + l: h keeps the top 8 significand bits (truncation), m the next
-// 8 of the remainder x - h (exact in fp32), l what is left (at most 8 bits: exact in bf16), exact
-// whenever |x| >= 2^-110 or x = 0. A bf16 weight times a part is exact in fp32, so the matrix cores
-// sum exact products: out = W h + W m + W l, with fp32 roundings only in the accumulation (a chain
-// of at most 3 K / 32 + 2 matrix operations and NW wave partials per output; the test bound is that
-// of K sequential fp32 additions). An int8 weight widens to bf16 exactly (|q| <= 127).
+// ---- matrix-core forms, from 3 or 4 rows up -----------------------------------------------------
+// The hidden rows are fp32 and v_mfma_f32_16x16x32_bf16 multiplies bf16, so each x is scaled by 2^32
+// and split exactly into three bf16 parts, 2^32 x = h + m + l: h keeps the top 8 significand bits
+// (truncation), m the next 8 of the remainder (exact in fp32), l what is left (at most 8 bits: exact in
+// bf16). The scale keeps every bit of the smallest x: unscaled, a part below bf16's last place of 2^-133
+// is cut short (x near 2^-120 then had 13 bits of 24); it costs one multiplication per x (256 x 1024 ->
+// 3072 10.35 -> 10.48 us, 4096 rows 89.9 -> 90.7). A bf16 weight times a part is exact in fp32, so
+// the matrix cores sum exact products: out = 2^-32 (W h + W m + W l), with fp32 roundings only in the
+// accumulation (each kernel says how its sums are kept short; the test bound is that of K sequential
+// fp32 additions). An int8 weight widens to bf16 exactly (|q| <= 127).
 //
 // +-inf and NaN need no care in the split: such an x (its remainders are NaN) or weight (inf times a
-// zero part is NaN) leaves NaN in its outputs, and an output that is not finite is formed again by
-// output_in_order, whose products and sums follow IEEE. Finite outputs had finite operands.
+// zero part is NaN) leaves NaN in its outputs, and so do an |x| or a sum of 2^96 and more, which the
+// scale takes out of range. An output that is not finite is formed again by output_in_order, whose
+// products and sums follow IEEE. Finite outputs had finite operands.
 //
 // MFMA operand layout (16x16x32): lane l supplies A[l % 16][8 (l / 16) + 0..7] and
 // B[8 (l / 16) + 0..7][l % 16], and holds C[4 (l / 16) + i][l % 16], i = 0..3. Here A = W (outputs by
 // k), B = x^T (k by rows), so lane l reads 8 consecutive k of one weight row and of one hidden row and
-// ends with four consecutive outputs of one hidden row. Tile rows past the last hidden row or output
-// read the last one (each result depends on its own row of A and column of B alone; what they
-// compute is not stored); past the end of k the hidden values are zero.
+// ends with four consecutive outputs of one hidden row. Tile rows past the last hidden row or output,
+// and entries past the end of k, read as zero (each result depends on its own row of A and column of B
+// alone; what they compute is not stored).
 typedef __bf16 bf8 __attribute__((ext_vector_type(8)));
+constexpr float kUp = 0x1p32f, kDown = 0x1p-32f;
 
-// three exact bf16 parts of 8 finite fp32 values
+// three exact bf16 parts of 8 fp32 values below 2^96, times kUp
 struct Parts {
     u4 h, m, l;
 };
@@ -234,8 +238,9 @@ __device__ __forceinline__ Parts split3(const f4& a, const f4& b) {
     uint32_t th[8], tm[8], tl[8];
 #pragma unroll
     for (int i = 0; i < 8; i++) {
-        th[i] = __float_as_uint(v[i]);
-        const float r1 = v[i] - __uint_as_float(th[i] & 0xFFFF0000u);
+        const float x = v[i] * kUp;
+        th[i] = __float_as_uint(x);
+        const float r1 = x - __uint_as_float(th[i] & 0xFFFF0000u);
         tm[i] = __float_as_uint(r1);
         tl[i] = __float_as_uint(r1 - __uint_as_float(tm[i] & 0xFFFF0000u));
     }
@@ -478,7 +483,7 @@ __global__ __launch_bounds__(64 * NW) void head_mfma_kernel(HeadArgs a, int row_
         double dsum = 0.0;
 #pragma unroll
         for (int w = 0; w < NH; w++) dsum += (double)sm.part[w][(nl / 16) * RT + rl / 16][l][nl % 4];
-        float sum = (float)dsum;
+        float sum = (float)(dsum * (double)kDown);
         const int n = n0 + nl, r = r0 + rl;
         if (n >= a.n || r >= a.rows) continue;
         if constexpr (I8) sum *= a.scale[n];
@@ -546,8 +551,9 @@ __global__ __launch_bounds__(kHT) __attribute__((amdgpu_waves_per_eu(2))) void h
             uint32_t th[4], tm[4], tl[4];
 #pragma unroll
             for (int i = 0; i < 4; i++) {
-                th[i] = __float_as_uint(xr[j][i]);
-                const float r1 = xr[j][i] - __uint_as_float(th[i] & 0xFFFF0000u);
+                const float x = xr[j][i] * kUp;
+                th[i] = __float_as_uint(x);
+                const float r1 = x - __uint_as_float(th[i] & 0xFFFF0000u);
                 tm[i] = __float_as_uint(r1);
                 tl[i] = __float_as_uint(r1 - __uint_as_float(tm[i] & 0xFFFF0000u));
             }
@@ -614,7 +620,7 @@ __global__ __launch_bounds__(kHT) __attribute__((amdgpu_waves_per_eu(2))) void h
         for (int q = 0; q < WR; q++) {
             const int r = r0 + rw + 16 * q + c16;
             float* o = a.out + (int64_t)r * a.ldo + n;
-            f4 v = tot[i][q] + low[i][q];
+            f4 v = (tot[i][q] + low[i][q]) * kDown;
 #pragma unroll
             for (int e = 0; e < 4; e++) {
                 if constexpr (I8) v[e] *= sc[e];
