@@ -9,6 +9,7 @@ import pytest
 from oracle import ref
 from parity import compare_ids
 from voxwerk_amd._lib import PARAMS_DTYPE
+from voxwerk_amd.hip import DeviceArray
 
 pytestmark = pytest.mark.gpu
 
@@ -104,6 +105,25 @@ def test_split_special_rows(ctx):
     ids = check(ctx, x, p, np.linspace(0.05, 0.95, rows), off, hist, label="special")
     assert ids[0] == vocab - 1 and ids[2] == -3 and ids[3] == 39999 and ids[6] == -3 and ids[7] == -3
     assert ids[8] == -2 and ids[9] == -2
+
+
+@pytest.mark.parametrize("top_k,top_p,do_sample", [(50, 1.0, 1), (0, 0.9, 1), (300, 0.9, 1), (0, 1.0, 0)])
+def test_split_reads_no_history_without_a_penalty(ctx, top_k, top_p, do_sample):
+    """Device calls whose rows have the penalty off and whose offsets were never filled (they point far past
+    the ids): nothing of the history is read, the ids are those of the call without one."""
+    rng = np.random.default_rng(top_k)
+    rows, vocab = 5, 30000
+    x = rng.standard_normal((rows, vocab)).astype(np.float32)
+    p = options(rng, rows, vocab, top_k=top_k, top_p=np.float32(top_p), do_sample=do_sample, rep_penalty=np.float32(1.0))
+    d_x, d_p, d_u = DeviceArray.from_numpy(x), DeviceArray.from_numpy(p), DeviceArray.from_numpy(rng.random(rows))
+    off = (np.arange(rows + 1) * 4096 + (1 << 30)).astype(np.int32)
+    d_off, d_ids, d_out = DeviceArray.from_numpy(off), DeviceArray.from_numpy(np.zeros(4, np.int32)), DeviceArray((rows,), np.int32)
+    ctx.sample_device(rows, vocab, d_x, vocab, d_p, 1, d_u, d_out)
+    ctx.synchronize()
+    want = d_out.numpy().copy()
+    ctx.sample_device(rows, vocab, d_x, vocab, d_p, 1, d_u, d_out, d_off, d_ids)
+    ctx.synchronize()
+    assert np.array_equal(d_out.numpy(), want)
 
 
 def test_split_resident_store_with_generators(ctx):

@@ -309,16 +309,18 @@ __device__ __forceinline__ SplitEnd split_row(const SampleArgs& a, int vec, int 
 #pragma unroll
         for (int j = 0; j < 4; j++) v[4 * c + j] = q[j];
     }
-    // the history range and its first ids are on their way before the options say whether they count
+    // A row without a penalty reads nothing of its history (a caller need not have filled it); with one,
+    // the first ids are on their way while the segment is.
+    const vxs_params P = a.params[(int64_t)r * a.params_stride];
+    const bool pen_on = P.rep_penalty != 1.0f && has_history(a);
     HistRange hr{0, 0};
-    if (has_history(a)) hr = history_range(a, r);
+    if (pen_on) hr = history_range(a, r);
     int first[kIdsAhead];
 #pragma unroll
     for (int k = 0; k < kIdsAhead; k++) {
         const int h = hr.h0 + k * kTW + g.t;
         first[k] = h < hr.h1 ? a.hist_ids[h] : 0;
     }
-    const vxs_params P = a.params[(int64_t)r * a.params_stride];
     const bool greedy = !P.do_sample;
     const double u = greedy ? 0.0 : readlane_d(row_uniform(a, r), 0);  // before any workgroup can end the row's step
     RowX X;
@@ -327,7 +329,7 @@ __device__ __forceinline__ SplitEnd split_row(const SampleArgs& a, int vec, int 
     X.rinv = 1.0f / P.rep_penalty;
     X.fastdiv = __builtin_fabsf(P.rep_penalty) >= 0x1p-60f && __builtin_fabsf(P.rep_penalty) <= 0x1p60f;
     bool bad_id = false;
-    if (P.rep_penalty != 1.0f && has_history(a)) {
+    if (pen_on) {
         bad_id = !build_segment_bitmap(g, a, hr, V, lo, L, first, bm_dyn);
         X.bm = bm_dyn - (lo >> 5);  // indexed by vocabulary entry
     }
