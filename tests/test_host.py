@@ -59,6 +59,16 @@ def test_params_struct_layout(tmp_path):
         assert _lib.PARAMS_DTYPE.fields[name][1] == int(off)
 
 
+def test_split_workspaces_over_streams(tmp_path):
+    """The workspaces of split wide rows, compiled over a HIP runtime that only keeps the order of work."""
+    exe = tmp_path / "split_workspace"
+    subprocess.run(["g++", "-std=c++17", "-O1", "-Wno-subobject-linkage", "-D__HIP_PLATFORM_AMD__",
+                    "-I", os.path.join(build.ROCM, "include"), "-I", build.INCLUDE,
+                    os.path.join(REPO, "tests", "split_workspace.cpp"), "-o", str(exe)], check=True)
+    p = subprocess.run([str(exe)], capture_output=True, text=True, timeout=60)
+    assert p.returncode == 0, p.stdout
+
+
 def test_hip_build_flags():
     flags = " ".join(build.HIP_FLAGS)
     assert "--offload-arch=gfx950" in flags

@@ -348,7 +348,11 @@ SplitWs* split_workspace(vxs_ctx* ctx, const vxs::SampleArgs& a) {
     SplitWs* w = nullptr;
     for (SplitWs& x : ctx->split_ext)
         if (x.p && x.stream == st) w = &x;
-    if (w) return idle(*w) || hipStreamWaitEvent(st, w->last, 0) == hipSuccess ? w : nullptr;
+    if (w) {
+        if (idle(*w) || hipStreamWaitEvent(st, w->last, 0) == hipSuccess) return w;
+        (void)hipGetLastError();
+        return nullptr;
+    }
     for (SplitWs& x : ctx->split_ext)
         if (!w && idle(x)) w = &x;
     if (!w) return nullptr;
@@ -365,10 +369,15 @@ SplitWs* split_workspace(vxs_ctx* ctx, const vxs::SampleArgs& a) {
 // Enqueue the sampler on the context's stream.
 hipError_t launch(vxs_ctx* ctx, const vxs::SampleArgs& a) {
     SplitWs* w = split_workspace(ctx, a);
-    hipError_t e = vxs::launch_sample(a, ctx->stream, w ? w->p : nullptr);
-    if (e == hipSuccess && w && w->last) {
-        e = hipEventRecord(w->last, ctx->stream);
-        w->recorded = true;
+    const hipError_t e = vxs::launch_sample(a, ctx->stream, w ? w->p : nullptr);
+    if (w && w->last) {
+        // Whatever the launch returned: that can be an older error of the program's, with the kernel (and
+        // a new workspace's clearing) queued all the same.
+        w->recorded = hipEventRecord(w->last, ctx->stream) == hipSuccess;
+        if (!w->recorded) {  // nothing would tell when the workspace is free again
+            (void)hipGetLastError();
+            if (hipStreamSynchronize(ctx->stream) != hipSuccess) (void)hipDeviceSynchronize();
+        }
     }
     return e;
 }
