@@ -9,7 +9,7 @@ import pytest
 from oracle import ref
 from parity import compare_ids
 from voxwerk_amd._lib import PARAMS_DTYPE
-from voxwerk_amd.hip import DeviceArray
+from voxwerk_amd.hip import DeviceArray, Event
 
 pytestmark = pytest.mark.gpu
 
@@ -81,6 +81,57 @@ def test_split_nucleus_ties_and_cuts(ctx, vocab):
             p = options(rng, rows, vocab, top_p=np.float32(top_p), top_k=k, rep_penalty=np.float32(1.0), temperature=np.float32(1.0))
             for u in (rng.random(rows), np.full(rows, 0.0), np.full(rows, 1.0 - 2.0**-53)):
                 check(ctx, x, p, u, label=f"ties V={vocab} p={top_p} k={k}")
+
+
+def topk_us(ctx, x, k):
+    """Device time of a call with this top-k, the best of several."""
+    rows, vocab = x.shape
+    p = np.zeros(rows, dtype=PARAMS_DTYPE)
+    p["do_sample"], p["top_k"], p["top_p"], p["temperature"], p["rep_penalty"] = 1, k, np.float32(0.95), 1.0, 1.0
+    p["keep_id"] = p["ban_id"] = -1
+    d_x, d_p, d_u = DeviceArray.from_numpy(x), DeviceArray.from_numpy(p), DeviceArray.from_numpy(np.full(rows, 0.4))
+    d_out, best = DeviceArray((rows,), np.int32), np.inf
+    for _ in range(8):
+        a, b = Event(), Event()
+        a.record(ctx.stream())
+        for _ in range(4):
+            ctx.sample_device(rows, vocab, d_x, vocab, d_p, 1, d_u, d_out)
+        b.record(ctx.stream())
+        b.synchronize()
+        best = min(best, 250 * a.elapsed_ms(b))
+    return best
+
+
+@pytest.mark.parametrize("rows,vocab", [(2, 20000), (16, 151936)])
+def test_split_topk_near_256_stays_split(ctx, rows, vocab):
+    """As k nears 256, the bound a segment gets from its 256 thread maxima lets more entries through than its
+    list holds. It is raised then: a row sampled again by one workgroup takes ten times as long and more."""
+    x = np.random.default_rng(vocab).standard_normal((rows, vocab)).astype(np.float32)
+    us = {k: topk_us(ctx, x, k) for k in (128, 245, 250, 254, 256)}
+    print(us, flush=True)
+    assert max(us.values()) < 4 * us[128]
+
+
+@pytest.mark.parametrize("vocab", [20000, 151936])
+@pytest.mark.parametrize("k", [60, 250, 256])
+def test_split_topk_bound_raised(ctx, vocab, k):
+    """Rows whose segments get more entries than the list from the first bound: over every magnitude, of both
+    signs, subnormal, with outliers, finite at few threads, large at few threads, tied."""
+    rng = np.random.default_rng(vocab + k)
+    x = rng.standard_normal((10, vocab))
+    i = np.arange(vocab)
+    x[1] = np.copysign(10.0 ** rng.uniform(-38, 38, vocab), x[1])
+    x[2] *= 1e-40
+    x[3, [5, vocab - 9]] = 2e38, -2e38
+    x[4, i % 1024 >= 20] = -np.inf
+    x[5, i % 1024 < 4 * k] += 30
+    x[6] = np.round(x[6] * 16) / 16
+    x[7] = np.where(rng.random(vocab) < 0.5, -1.0, -0.0)
+    x[8] = -np.abs(x[8])
+    x = x.astype(np.float32)
+    p = options(rng, 10, vocab, top_k=k, top_p=np.float32(0.95), rep_penalty=np.float32(1.0), supp_begin=0, supp_end=0)
+    for u in (rng.random(10), rng.random(10)):
+        check(ctx, x, p, u, label=f"raised V={vocab} k={k}")
 
 
 def test_split_special_rows(ctx):

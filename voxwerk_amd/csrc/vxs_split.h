@@ -48,7 +48,7 @@ struct alignas(64) SplitRow {  // zero between calls
 };
 struct alignas(16) SplitSeg {
     uint32_t maxkey, cnt, bad, n;     // largest key; finite entries; 1 non-finite, 2 bad history id; entries listed
-    uint32_t bkey, argi, kmin, kmax;  // top-k: a key with ceil(k/S) entries at or above; greedy: index; keys of the cut's part
+    uint32_t bkey, argi, kmin, kmax;  // top-k: a key with the segment's share of k entries at or above; greedy: index; keys of the cut's part
     uint64_t kept, pad;
     union {
         uint64_t list[kSegList];      // top-k: key << 32 | index, in index order
@@ -168,7 +168,7 @@ __device__ __forceinline__ bool split_topk_finish(const SampleArgs& a, int vec, 
         if (g.t == 0) put_id(a, r, a.vocab - 1);
         return false;
     }
-    if (__ballot(my_n > (uint32_t)kSegList)) return true;  // a list overflowed (ties)
+    if (__ballot(my_n > (uint32_t)kSegList)) return true;  // more entries than a list holds: ties, mostly
     uint32_t* wkey = s.wkey[g.wv];
     int32_t* widx = s.widx[g.wv];
     int wn = 0;
@@ -426,25 +426,49 @@ __device__ __forceinline__ SplitEnd split_row(const SampleArgs& a, int vec, int 
     const uint32_t cnt = (uint32_t)g.combine(fin, [](uint64_t p, uint64_t q) { return p + q; });
 
     if (K > 0 && K <= kKMax && K < V) {
-        // ---- top-k: this segment's entries at or above a lower bound of its k-th largest: the k-th
-        // largest of the thread maxima (all finite ones when there are at most k)
+        // ---- top-k: this segment's entries at or above a lower bound of its k-th largest (all finite ones
+        // when there are at most k): the k-th largest of the thread maxima. As k nears their number the bound
+        // falls to the least of them and the list overflows, at once for k from 250 on; two maxima per
+        // thread, of the even and of the odd sweeps, keep it. Their search takes 2 us more, which rows of many
+        // segments get back from shorter lists (us, one / two: 16 x 151936 k = 150 34.9 / 34.3, 200 43.8 / 38.8,
+        // 240 62 / 44, 256 182 / 48; 64 x 20000 k = 200 24.6 / 27.4, 240 29.3 / 28.6, 256 82 / 29.4; 1 x 8193
+        // k = 200 22.1 / 24.2, 240 23.1 / 25.1, 256 55 / 25.6).
+        // this segment's share of k by length: the shares add up to k and more, and a short last segment's
+        // is no harder to reach than the others' (64 x 9001, the same share for all: k = 50 17.1 -> 16.6, 240 28.6 -> 27.6)
+        const int Kq = (K * (hi - lo) + V - 1) / V;
+        float Tb = kNegInf;
+        uint32_t bq = 0;  // a key of which at least Kq entries of this segment are at or above (0: fewer are finite)
         float* tm = reinterpret_cast<float*>(&s.wkey[0][0]);
-        tm[g.t] = tmx;
-        __syncthreads();
-        uint32_t mk[kTW / 64];
-        uint32_t mlo = 0xffffffffu, mhi = 0;
+        auto bounds = [&](auto per_thread) {
+            constexpr int N = decltype(per_thread)::value * kTW / 64;
+            __syncthreads();
+            uint32_t mk[N];
+            uint32_t mlo = 0xffffffffu, mhi = 0;
 #pragma unroll
-        for (int q = 0; q < kTW / 64; q++) {
-            mk[q] = f2key(tm[g.lane + 64 * q]);
-            mlo = min(mlo, mk[q]);
-            mhi = max(mhi, mk[q]);
+            for (int q = 0; q < N; q++) {
+                mk[q] = f2key(tm[g.lane + 64 * q]);
+                mlo = min(mlo, mk[q]);
+                mhi = max(mhi, mk[q]);
+            }
+            mlo = wave_umin(mlo);
+            mhi = wave_umax(mhi);
+            if (cnt > (uint32_t)K) Tb = key2f(wave_bound_regs4(mk, mlo, mhi, K, 8));
+            if (cnt >= (uint32_t)Kq) bq = wave_bound_regs4(mk, mlo, mhi, Kq, 4);
+        };
+        if (K <= (S > 5 ? 192 : 240)) {
+            tm[g.t] = tmx;
+            bounds(std::integral_constant<int, 1>());
+        } else {
+            float odd = kNegInf;
+            tmx = kNegInf;
+#pragma unroll
+            for (int c = 0; c < NC; c++)
+#pragma unroll
+                for (int j = 0; j < 4; j++) (c & 1 ? odd : tmx) = fmaxf(c & 1 ? odd : tmx, v[4 * c + j]);
+            tm[g.t] = tmx;
+            tm[kTW + g.t] = odd;
+            bounds(std::integral_constant<int, 2>());
         }
-        mlo = wave_umin(mlo);
-        mhi = wave_umax(mhi);
-        const int Kq = (K + S - 1) / S;
-        const float Tb = cnt > (uint32_t)K ? key2f(wave_bound_regs4(mk, mlo, mhi, K, 8)) : kNegInf;
-        // a key of which at least Kq entries of this segment are at or above (0: fewer are finite)
-        const uint32_t bq = cnt >= (uint32_t)Kq ? wave_bound_regs4(mk, mlo, mhi, Kq, 4) : 0u;
         constexpr int NH = (NC + 3) / 4;
         uint64_t excl[NH], totals[NH];
         uint32_t tot = 0;

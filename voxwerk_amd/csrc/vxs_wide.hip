@@ -1473,11 +1473,19 @@ size_t split_workspace_bytes() { return (sizeof(SplitRow) + sizeof(SplitSeg)) * 
 
 // Rows over several workgroups (vxs_split.h): the sweeps of 1024 entries per segment, 0 when the call is not
 // for it. Segments of 4096 entries while the call then has at most 1024 of them (four workgroups per
-// compute unit, all resident), else of 10240; one workgroup per row when the call writes back, or has
-// rows enough to keep the compute units busy that way (us, split / one workgroup per row, top-k 50 or as
-// said: 1 x 151936 19.9 / 74, 16 x 151936 22.1 / 76, 64 32.8 / 78, 136 51.3 / 79, 200 x 20000 26.6 / 28.4,
-// 300 x 20000 31.8 / 29.9, 128 x 151936 at top-k 200 70 / 86; nucleus, top-p 0.9: 4 x 151936 25.6 / 1017, 64
-// 45.7 / 1361, 128 82 / 1385, 300 x 20000 40.7 / 220; top-k 400: 16 x 151936 48 / 1386, 2 x 30000 31 / 289).
+// compute unit), else of 10240; one workgroup per row when the call writes back, or has rows enough to keep
+// the compute units busy that way. The options are in device memory, so one limit serves them all, at the
+// rows where top-k up to about 150 still gains (us, split / one workgroup per row; nucleus top-p 0.9):
+//                 top-k 50       100         200         240         256         nucleus     greedy
+//   1 x 151936    16.3 / 70    28 / 68     35 / 74     39 / 75     43 / 80     24 / 655    5.4 / 44
+//   16 x 151936   19.2 / 74    30 / 75     39 / 79     44 / 83     48 / 84     30 / 848    5.8 / 45
+//   136 x 151936  40 / 76      47 / 76     72 / 82     74 / 86     81 / 88     79 / 958    18.5 / 45
+//   192 x 40000   23.8 / 34    27.8 / 36.6 33.6 / 43   39 / 44.7   37 / 45     36 / 241    8.8 / 14.8
+//   192 x 20000   20.6 / 25.3  24.2 / 28.3 29.6 / 32   36.6 / 33.9 36.7 / 34.2 24.7 / 123  6.2 / 9.1
+//   192 x 9001    18.7 / 20.6  22.4 / 22.9 27.9 / 26.7 29.0 / 28.2 32.9 / 28.5 22.8 / 63   5.8 / 6.0
+//   64 x 9001     16.6 / 20.4  19.8 / 22.8 24.2 / 26.5 27.6 / 28.0 30.9 / 28.4 21.0 / 63   5.5 / 6.0
+// (300 x 20000: top-k 50 31.8 / 29.9, nucleus 40.7 / 220). On a caller's stream the workspace's event adds
+// 1.0 to 1.3 us (64 x 9001 greedy 6.7).
 static int split_segment(const SampleArgs& a) {
     if (a.rows > 192 || a.out_logits || a.out_probs || (a.kflags & KF_STOP_AFTER_PENALTY)) return 0;
     for (int nc : {4, 10}) {
