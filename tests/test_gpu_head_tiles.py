@@ -8,6 +8,7 @@ import pytest
 
 from oracle.head_np import head_bound, head_exact, head_int8_bound, head_int8_exact, pack_int8
 from test_gpu_head import _bf16, _run, _run_int8
+from voxwerk_amd.hip import DeviceArray, Event
 
 pytestmark = pytest.mark.gpu
 
@@ -38,17 +39,22 @@ def test_head_tiles_within_bound(ctx, rows, k, n, pad, int8):
     assert np.all(err <= bound), f"max err/bound {np.max(err / bound):.3f}"
 
 
-@pytest.mark.parametrize("rows,k,n", [(5, 1024, 600), (256, 512, 3072), (400, 72, 2050)])
-def test_head_tiles_nonfinite(ctx, rows, k, n):
+@pytest.mark.parametrize("int8", [False, True])
+@pytest.mark.parametrize("rows,k,n", [(5, 1024, 600), (256, 512, 3072), (400, 72, 2050), (1100, 264, 3001)])
+def test_head_tiles_nonfinite(ctx, rows, k, n, int8):
     """A hidden row with +inf, one with NaN, one with both infinities; a weight row with -inf, one with
-    NaN, one with zeros where the infinities meet it (0 * inf = NaN)."""
+    NaN (bf16), one with zeros where the infinities meet it (0 * inf = NaN)."""
     rng = np.random.default_rng(rows + k)
     x = rng.standard_normal((rows, k)).astype(np.float32)
     wf = (rng.standard_normal((n, k)) * 0.05).astype(np.float32)
     x[0, 3], x[rows - 1, k - 1], x[2, 5], x[2, 6] = np.inf, np.nan, np.inf, -np.inf
-    wf[1, 9], wf[n - 1, k - 2], wf[4, 3] = -np.inf, np.nan, 0.0
-    got = _run(ctx, x, _bf16(wf))
-    wd = (_bf16(wf).astype(np.uint32) << 16).view(np.float32)
+    wf[4, 3] = 0.0
+    if int8:
+        q, scale = pack_int8(_bf16(wf))
+        got, wd = _run_int8(ctx, x, q, scale), q * scale[:, None]
+    else:
+        wf[1, 9], wf[n - 1, k - 2] = -np.inf, np.nan
+        got, wd = _run(ctx, x, _bf16(wf)), (_bf16(wf).astype(np.uint32) << 16).view(np.float32)
     with np.errstate(invalid="ignore"):  # elementwise products and a plain sum, no library shortcuts
         for r in (0, 1, 2, rows - 1):
             want = (x[r].astype(np.float64) * wd.astype(np.float64)).sum(axis=1)
@@ -58,3 +64,34 @@ def test_head_tiles_nonfinite(ctx, rows, k, n):
             want = (x.astype(np.float64) * wd[c].astype(np.float64)).sum(axis=1)
             for cls in (np.isnan, np.isposinf, np.isneginf):
                 assert np.array_equal(cls(got[:, c]), cls(want)), (c, cls)
+
+
+def head_us(ctx, x, n):
+    rows, k = x.shape
+    w = _bf16(np.random.default_rng(n).standard_normal((n, k)) * 0.05)
+    d_x, d_w, d_o = DeviceArray.from_numpy(x), DeviceArray.from_numpy(w), DeviceArray((rows, n), np.float32)
+    best = np.inf
+    for _ in range(8):
+        a, b = Event(), Event()
+        a.record(ctx.stream())
+        for _ in range(4):
+            ctx.head_device(rows, k, n, d_x, k, d_w, k, d_o, n)
+        b.record(ctx.stream())
+        b.synchronize()
+        best = min(best, 250 * a.elapsed_ms(b))
+    return best
+
+
+@pytest.mark.parametrize("rows,k,n", [(24, 1024, 2048), (256, 1024, 3072), (4096, 1024, 3072)])
+def test_head_nonfinite_rows_cost_little(ctx, rows, k, n):
+    """One hidden row of NaN (a finished sequence's slot, say) or with an infinity, and NaN in every row,
+    against the finite call."""
+    x = np.random.default_rng(rows).standard_normal((rows, k)).astype(np.float32)
+    us = {"finite": head_us(ctx, x, n)}
+    for name, r, c, v in (("NaN row", rows // 2, slice(None), np.nan), ("one NaN", rows // 2, k - 1, np.nan),
+                          ("one inf", rows // 2, 7, np.inf), ("all rows", slice(None), k - 1, np.nan)):
+        bad = x.copy()
+        bad[r, c] = v
+        us[name] = head_us(ctx, bad, n)
+    print(us, flush=True)
+    assert max(us.values()) < 2 * us["finite"] + 10

@@ -217,7 +217,7 @@ __global__ __launch_bounds__(kHT) void head_i8_kernel(HeadArgs a) {
 //
 // +-inf and NaN need no care in the split: such an x (its remainders are NaN) or weight (inf times a
 // zero part is NaN) leaves NaN in its outputs, and so do an |x| or a sum of 2^96 and more, which the
-// scale takes out of range. An output that is not finite is formed again by output_in_order, whose
+// scale takes out of range. An output that is not finite is formed again on the VALU (redo_rows), whose
 // products and sums follow IEEE. Finite outputs had finite operands.
 //
 // MFMA operand layout (16x16x32): lane l supplies A[l % 16][8 (l / 16) + 0..7] and
@@ -313,6 +313,12 @@ __device__ __forceinline__ void wave_order() {
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
+// The workgroup meets and sees each other's LDS writes; global stores are not waited for.
+__device__ __forceinline__ void lds_barrier() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
 
 template <bool I8>
 __device__ __forceinline__ bf8 w_operand(const WRaw<I8>& r) {
@@ -322,24 +328,80 @@ __device__ __forceinline__ bf8 w_operand(const WRaw<I8>& r) {
         return __builtin_bit_cast(bf8, r);
 }
 
-// One output in k order by fp32 FMAs, the int8 scale last: for results that are not finite.
-template <bool I8>
-__device__ __forceinline__ float output_in_order(const HeadArgs& a, int r, int n) {
-    const float* x = a.x + (int64_t)r * a.ldx;
-    float acc = 0.0f;
-#pragma unroll 1
-    for (int k = 0; k < a.k; k++) {
-        float w;
-        if constexpr (I8)
-            w = (float)(int)a.q[(int64_t)n * a.ldw + k];
-        else
-            w = __uint_as_float((uint32_t)a.w[(int64_t)n * a.ldw + k] << 16);
-        acc = __builtin_fmaf(w, x[k], acc);
-    }
-    if constexpr (I8) acc *= a.scale[n];
-    return acc;
-}
 __device__ __forceinline__ bool finite(float v) { return __builtin_fabsf(v) < __builtin_huge_valf(); }
+
+// The outputs that are not finite among the `cols` from n0 on of the tile rows `rows` (a bit each), formed
+// again as the VALU form does, by a workgroup whose waves have stored theirs (`lds`: two words that are free
+// once it has met). A row with a NaN is done, as its outputs are NaN: the waves look through a row each. Of
+// the others' outputs the waves (a power of two) take four each, the lanes along k, so that their loads are in
+// flight together. (us, finite / one row with a NaN / one with an infinity / a NaN in every row; before, each lane
+// formed its own outputs in k order: 24 x 1024 -> 2048 4.4 / 5.7 / 7.9 / 8.3, before 4.4 / 74 / 74 / 121; 256 x
+// 1024 -> 3072 11.4 / 13.8 / 18.9 / 26.6, before 11.4 / 95 / 95 / 1411; 4096 rows 96 / 97 / 110 / 145, before 97 /
+// 1230 / 1230 / 22460.)
+template <bool I8>
+__device__ __forceinline__ void redo_rows(const HeadArgs& a, int r0, int n0, int cols, uint64_t rows, uint32_t* lds, int wv, int nwaves,
+                                          int lane) {
+    const int end = min(n0 + cols, a.n);
+    __syncthreads();
+    if (threadIdx.x < 2) lds[threadIdx.x] = (uint32_t)(rows >> (32 * threadIdx.x));
+    __syncthreads();
+#pragma unroll 1
+    for (uint64_t left = rows; left; left &= left - 1) {
+        const int row = (int)__builtin_ctzll(left);
+        if ((row & (nwaves - 1)) != wv) continue;
+        const float* x = a.x + (int64_t)(r0 + row) * a.ldx;
+        bool nan = false;
+#pragma unroll 1
+        for (int k = 4 * lane; k < a.k; k += 256) {
+            const f4 v = *reinterpret_cast<const f4*>(x + k);
+            nan = nan || v.x != v.x || v.y != v.y || v.z != v.z || v.w != v.w;
+        }
+        if (__ballot(nan) && lane == 0) atomicAnd(&lds[row >> 5], ~(1u << (row & 31)));
+    }
+    __syncthreads();
+#pragma unroll 1
+    for (rows = lds[0] | (uint64_t)lds[1] << 32; rows; rows &= rows - 1) {
+        const int row = (int)__builtin_ctzll(rows), r = r0 + row;
+        const float* x = a.x + (int64_t)r * a.ldx;
+        float* o = a.out + (int64_t)r * a.ldo;
+        uint64_t bad[2];  // a bit per output (of which this wave's own are not changing)
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            const int n = n0 + 64 * h + lane;
+            bad[h] = __ballot(n < end && !finite(o[min(n, end - 1)]));
+        }
+#pragma unroll 1
+        for (int g = 0; 4 * g < cols; g++) {
+            const uint32_t four = (uint32_t)(bad[g >> 4] >> (4 * (g & 15))) & 15u;
+            if (!four || ((g + row) & (nwaves - 1)) != wv) continue;
+            const int n = n0 + 4 * g;
+            float acc[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+            for (int k = 8 * lane; k < a.k; k += 512) {
+                const f4 xa = *reinterpret_cast<const f4*>(x + k), xb = *reinterpret_cast<const f4*>(x + k + 4);
+                WRaw<I8> w[4];
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    const int64_t at = (int64_t)min(n + j, end - 1) * a.ldw + k;
+                    if constexpr (I8)
+                        w[j] = *reinterpret_cast<const u2*>(a.q + at);
+                    else
+                        w[j] = *reinterpret_cast<const u4*>(a.w + at);
+                }
+#pragma unroll
+                for (int j = 0; j < 4; j++) acc[j] = dot8(__builtin_bit_cast(u4, w_operand<I8>(w[j])), xa, xb, acc[j]);
+            }
+#pragma unroll
+            for (int mask = 32; mask >= 1; mask /= 2)
+#pragma unroll
+                for (int j = 0; j < 4; j++) acc[j] += __shfl_xor(acc[j], mask);
+            if (lane < 4 && (four >> lane & 1u)) {
+                const float sum = lane == 0 ? acc[0] : lane == 1 ? acc[1] : lane == 2 ? acc[2] : acc[3];
+                o[n + lane] = I8 ? sum * a.scale[n + lane] : sum;
+            }
+        }
+    }
+}
 
 // XCD-aware tile order: workgroups go to the 8 XCDs in turn, each with an L2 of its own, so workgroup
 // b takes tile (b % 8) * per + b / 8 of the column-major tile list (row tiles fastest): an XCD's
@@ -368,7 +430,10 @@ __global__ __launch_bounds__(64 * NW) void head_mfma_kernel(HeadArgs a, int row_
     };
     __shared__ union {
         Turn turn[NW];
-        f4 part[NH][RT * CT][64];
+        struct {
+            f4 part[NH][RT * CT][64];
+            uint32_t redo;  // tile rows with an output that is not finite
+        };
     } sm;
     int rt, ct;
     if (!xcd_tile(row_tiles, tiles, rt, ct)) return;
@@ -464,6 +529,7 @@ __global__ __launch_bounds__(64 * NW) void head_mfma_kernel(HeadArgs a, int row_
         }
     }
     __syncthreads();  // every wave is done with its operand buffers
+    if (threadIdx.x == 0) sm.redo = 0;
     if (wv >= NH)
 #pragma unroll
         for (int t = 0; t < CT; t++)
@@ -487,9 +553,12 @@ __global__ __launch_bounds__(64 * NW) void head_mfma_kernel(HeadArgs a, int row_
         const int n = n0 + nl, r = r0 + rl;
         if (n >= a.n || r >= a.rows) continue;
         if constexpr (I8) sum *= a.scale[n];
-        if (!finite(sum)) sum = output_in_order<I8>(a, r, n);
+        if (!finite(sum)) atomicOr(&sm.redo, 1u << rl);
         a.out[(int64_t)r * a.ldo + n] = sum;
     }
+    lds_barrier();
+    const uint32_t rows = sm.redo;
+    if (__builtin_expect(rows != 0, 0)) redo_rows<I8>(a, r0, n0, 16 * CT, rows, reinterpret_cast<uint32_t*>(&sm.part), wv, NW, lane);
 }
 
 template <int RT, int CT, int NW>
@@ -607,7 +676,7 @@ __global__ __launch_bounds__(kHT) __attribute__((amdgpu_waves_per_eu(2))) void h
         __syncthreads();
     }
     const bool vec = a.ldo % 4 == 0 && ((uintptr_t)a.out & 15u) == 0;
-    bool fin = true;
+    bool bad[WR] = {};
 #pragma unroll
     for (int i = 0; i < WC; i++) {
         const int n = n0 + nw + 16 * i + 4 * g;
@@ -624,7 +693,7 @@ __global__ __launch_bounds__(kHT) __attribute__((amdgpu_waves_per_eu(2))) void h
 #pragma unroll
             for (int e = 0; e < 4; e++) {
                 if constexpr (I8) v[e] *= sc[e];
-                fin = fin && finite(v[e]);
+                bad[q] = bad[q] || !finite(v[e]);
             }
             if (r >= a.rows) continue;
             if (vec && n + 3 < a.n) {
@@ -636,15 +705,18 @@ __global__ __launch_bounds__(kHT) __attribute__((amdgpu_waves_per_eu(2))) void h
             }
         }
     }
-    if (fin) return;
-    // this lane's outputs once more: those that are not finite are formed in k order
-#pragma unroll 1
-    for (int e = 0; e < WC * WR * 4; e++) {
-        const int n = n0 + nw + 16 * (e / (4 * WR)) + 4 * g + e % 4, r = r0 + rw + 16 * (e / 4 % WR) + c16;
-        if (n >= a.n || r >= a.rows) continue;
-        float* o = a.out + (int64_t)r * a.ldo + n;
-        if (!finite(*o)) *o = output_in_order<I8>(a, r, n);
+    // each wave's rows with an output that is not finite, in LDS (the operands are done with)
+    uint32_t mine = 0;
+#pragma unroll
+    for (int q = 0; q < WR; q++) {
+        const uint64_t m = __ballot(bad[q] && r0 + rw + 16 * q + c16 < a.rows);
+        mine |= (uint32_t)((m | m >> 16 | m >> 32 | m >> 48) & 0xffffu) << (16 * q);
     }
+    uint32_t* redo = reinterpret_cast<uint32_t*>(&xs[0][0][0]);
+    if (lane == 0) redo[wv] = mine;
+    lds_barrier();
+    const uint64_t rows = (uint64_t)(redo[0] | redo[2]) | (uint64_t)(redo[1] | redo[3]) << (16 * WR);
+    if (__builtin_expect(rows != 0, 0)) redo_rows<I8>(a, r0, n0, BN, rows, redo, wv, 4, lane);
 }
 
 template <int WR, int WC>
