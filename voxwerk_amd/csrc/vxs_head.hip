@@ -790,7 +790,9 @@ hipError_t launch_head(const HeadArgs& a, hipStream_t stream) {
     if (a.k <= 0 || a.k > 2048) return hipErrorInvalidValue;
     // One to three rows (two above k = 1024) on the VALU: one pass over the weight with no operand to
     // turn, 1 x 1024 -> 2048 2.5 us (split-K form 3.9), 3 x 1024 -> 2048 3.6 (3.9), but 4 x 1024 -> 3072
-    // 4.5 (4.1) and 3 x 2048 -> 3072 6.2 (5.0). (bf16, back to back, 6 weights in turn; int8 alike.)
+    // 4.5 (4.1) and 3 x 2048 -> 3072 6.2 (5.0). (bf16, back to back, 6 weights in turn; int8 alike up to
+    // k = 1024. Above, int8 calls of at most 8192 outputs are 0.1 to 0.9 us faster on the VALU (4 x 2048 -> 512 4.5,
+    // here 5.2; 12 x 2048 -> 64 4.3, 5.1), but with a rounding error of 1.0e-7 where this form's is 0.7e-7.)
     const bool few = a.rows <= 2 || (a.rows == 3 && a.k <= 1024);
     if (!few && mfma_fits(a)) {
         // The split-K form with the smallest tile that leaves at most one workgroup per compute unit:
