@@ -96,6 +96,13 @@ VXS_API int vxs_set_stream(vxs_ctx* ctx, void* hip_stream);
 VXS_API void* vxs_get_stream(const vxs_ctx* ctx);
 
 /*
+ * The longest time, in units of 10 ns, that the workgroups of a row split over several of them
+ * (vxs_sample_device) wait for each other before one samples it alone; 50000 (500 us) in a new
+ * context. The ids are the same. 0 gives every such wait up, for tests of that path.
+ */
+VXS_API int vxs_set_split_wait(vxs_ctx* ctx, uint32_t ticks);
+
+/*
  * Host-pointer sampling call; synchronous.
  * Replaces, for each row: Sampler.ApplyRepetitionPenalty (Sampler.cs:25-33), the suppression
  * loops (TalkerGenerator.cs:247-248, :371-372) and Sampler.Select (Sampler.cs:35-88) as

@@ -205,6 +205,51 @@ def test_split_resident_store_with_generators(ctx):
     store.close()
 
 
+@pytest.mark.parametrize("ticks", [0, 30, 100, 300, 1000])
+def test_split_meetings_given_up(ticks):
+    """Workgroups that wait for each other for too short a time (10 ns a tick; none at all at 0) give the row
+    up at one meeting or another, and one samples it alone: the same ids, histories and generators; and the
+    workspace, with normal waits again, serves the next call."""
+    from voxwerk_amd.sampler import Context
+
+    rng = np.random.default_rng(ticks)
+    rows, vocab = 24, 70000
+    p = options(rng, rows, vocab, temperature=np.float32(1.0))
+    p["top_k"], p["top_p"] = [0, 0, 300, 40000, 0, 50] * 4, np.float32([0.9, 1.0, 0.9, 1.0, 0.3, 0.9] * 4)
+    hists = [rng.integers(0, vocab, 5).astype(np.int32) for _ in range(rows)]
+    logits = [(rng.standard_normal((rows, vocab)) * 2).astype(np.float32) for _ in range(3)]
+    out = []
+    for wait in (ticks, 50000):
+        with Context(0) as c:
+            store = c.history(rows, 64)
+            for r in range(rows):
+                store.set(r, hists[r])
+                store.seed(r, 100 + r)
+            ids = []
+            for x in logits:
+                for w in (wait, 50000):
+                    assert c._lib.vxs_set_split_wait(c.handle, w) == 0
+                    ids.append(c.sample_batch(store, x, np.arange(rows), p, None, append=True, rng="talker"))
+            if wait == 0:  # the path is taken: one workgroup per row takes many times as long
+                d = [DeviceArray.from_numpy(v) for v in (logits[0], p)] + [DeviceArray((rows,), np.int32)]
+                us = []
+                for w in (0, 50000):
+                    c._lib.vxs_set_split_wait(c.handle, w)
+                    a, b = Event(), Event()
+                    a.record(c.stream())
+                    for _ in range(4):
+                        c.sample_device(rows, vocab, d[0], vocab, d[1], 1, None, d[2])
+                    b.record(c.stream())
+                    b.synchronize()
+                    us.append(250 * a.elapsed_ms(b))
+                print(us, flush=True)
+                assert us[0] > 3 * us[1]
+            out.append((np.array(ids), [list(store.get(r)) for r in range(rows)], [list(store.draw(r, "talker", 3)) for r in range(rows)]))
+            store.close()
+    assert np.array_equal(out[0][0], out[1][0])
+    assert out[0][1:] == out[1][1:]
+
+
 def test_split_on_callers_streams_and_in_a_graph():
     import os
     import subprocess

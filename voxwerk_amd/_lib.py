@@ -88,6 +88,7 @@ _SIGNATURES = {
     "vxs_version": (c_char_p, []),
     "vxs_set_stream": (c_int, [c_void_p, c_void_p]),
     "vxs_get_stream": (c_void_p, [c_void_p]),
+    "vxs_set_split_wait": (c_int, [c_void_p, c_uint32]),
     "vxs_sample": (c_int, [c_void_p, c_int, c_int, _P, c_int64, _P, _P, _P, c_int, _P, _P, _P, _P, c_uint32]),
     "vxs_sample_device": (c_int, [c_void_p, c_int, c_int, _P, c_int64, _P, _P, _P, c_int, _P, _P, _P, _P, c_uint32]),
     "vxs_sample_noalloc": (c_int, [c_void_p, c_int, c_int, _P, c_int64, _P, _P, _P, c_int, _P, _P, c_uint32]),

@@ -105,6 +105,7 @@ struct vxs_ctx {
     void* noalloc = nullptr;  // this device's fixed scratch (vxs_sample_noalloc), looked up at create
     SplitWs split_own;                  // for own_stream, which outlives every use
     SplitWs split_ext[kSplitStreams];  // for streams set by the caller
+    uint32_t meet_ticks = vxs::kMeetTicks;
 };
 
 struct vxs_history {
@@ -367,7 +368,8 @@ SplitWs* split_workspace(vxs_ctx* ctx, const vxs::SampleArgs& a) {
 }
 
 // Enqueue the sampler on the context's stream.
-hipError_t launch(vxs_ctx* ctx, const vxs::SampleArgs& a) {
+hipError_t launch(vxs_ctx* ctx, vxs::SampleArgs& a) {
+    a.meet_ticks = ctx->meet_ticks;
     SplitWs* w = split_workspace(ctx, a);
     const hipError_t e = vxs::launch_sample(a, ctx->stream, w ? w->p : nullptr);
     if (w && w->last) {
@@ -655,6 +657,12 @@ VXS_API const char* vxs_last_error(const vxs_ctx* ctx) { return ctx ? ctx->err.c
 VXS_API int vxs_set_stream(vxs_ctx* ctx, void* hip_stream) {
     if (!ctx) return VXS_ERR_INVALID_ARG;
     ctx->stream = hip_stream ? static_cast<hipStream_t>(hip_stream) : ctx->own_stream;
+    return VXS_OK;
+}
+
+VXS_API int vxs_set_split_wait(vxs_ctx* ctx, uint32_t ticks) {
+    if (!ctx) return VXS_ERR_INVALID_ARG;
+    ctx->meet_ticks = ticks;
     return VXS_OK;
 }
 

@@ -69,7 +69,9 @@ struct SampleArgs {
     int direct_h0, direct_h1;
     double direct_u;
     vxs_params direct_params;
+    uint32_t meet_ticks;  // split wide rows: the longest wait of a row's workgroups for each other (10 ns each)
 };
+constexpr uint32_t kMeetTicks = 50000;  // its default, 500 us
 
 enum : int {
     kPathBlock = 0,  // one 256-thread workgroup per row

@@ -25,7 +25,7 @@
 // not above 0) are sampled by the last workgroup to leave, with the general algorithm.
 //
 // A meeting is a bounded wait: workgroups are dispatched in order, so a row's arrive together unless
-// other work holds the chip, and one that has waited kMeetTicks gives the row up for all its workgroups
+// other work holds the chip, and one that has waited meet_ticks gives the row up for all its workgroups
 // (a compare-and-swap that only succeeds while the meeting is incomplete, so they agree); the last to
 // leave then samples it. Nothing waits for that.
 
@@ -37,7 +37,6 @@ constexpr int kSegPart = 256;                           // entries of the cut's 
 constexpr int kRowPart = 768;                           // ... and per row
 constexpr int kMine = 4096;                             // indices of the cut's part kept in LDS per segment
 constexpr int kFineMass = kCoarse * 16;                 // LDS histogram: 64 buckets per octave
-constexpr uint64_t kMeetTicks = 50000;                  // 500 us of the 100 MHz counter
 constexpr uint32_t kAbandoned = 0x80000000u;
 
 struct alignas(64) SplitRow {  // zero between calls
@@ -85,14 +84,14 @@ __device__ __forceinline__ bool arrive_last(uint32_t* w, int S, const BlkW& g, W
     return s.wcomp[0] != 0;
 }
 // All S workgroups of the row (true), or the row was given up (false for all of them).
-__device__ __forceinline__ bool meet(uint32_t* w, int S, const BlkW& g, WideSmem& s) {
+__device__ __forceinline__ bool meet(uint32_t* w, int S, uint32_t ticks, const BlkW& g, WideSmem& s) {
     published();
     if (g.t == 0) {
         uint32_t cur = __hip_atomic_fetch_add(w, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         cur = cur & kAbandoned ? cur : cur + 1;
         const uint64_t t0 = __builtin_amdgcn_s_memrealtime();
         while (!(cur & kAbandoned) && cur != (uint32_t)S) {
-            if (__builtin_amdgcn_s_memrealtime() - t0 > kMeetTicks) {
+            if (__builtin_amdgcn_s_memrealtime() - t0 > ticks) {
                 if (__hip_atomic_compare_exchange_strong(w, &cur, cur | kAbandoned, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
                                                          __HIP_MEMORY_SCOPE_AGENT))
                     cur |= kAbandoned;
@@ -524,7 +523,7 @@ __device__ __forceinline__ SplitEnd split_row(const SampleArgs& a, int vec, int 
         }
     }
     const bool in = g.lane < S;  // lane l of every wave reads segment l's record
-    if (!meet(&row.meet[0], S, g, s)) return kEndUnsampled;
+    if (!meet(&row.meet[0], S, a.meet_ticks, g, s)) return kEndUnsampled;
     float mx;
     bool count_first;  // top-k above kKMax: the k-th largest first, by the same stages over counts
     {
@@ -616,7 +615,7 @@ __device__ __forceinline__ SplitEnd split_row(const SampleArgs& a, int vec, int 
             for (int i = 0; i < 16; i++) own += lds64[16 * g.t + ((i + g.t) & 15)];
             if (own) sum_up(row.coarse[stage][g.t], own);
         }
-        if (!meet(&meets[0], S, g, s)) return false;
+        if (!meet(&meets[0], S, a.meet_ticks, g, s)) return false;
         // the bucket where the ascending cumulative mass crosses T
         auto crossing = [&](uint64_t h, double rest, double& below, double& total) -> int {
             const double run = g.excl((double)h, total);
@@ -656,7 +655,7 @@ __device__ __forceinline__ SplitEnd split_row(const SampleArgs& a, int vec, int 
         __syncthreads();
         own = g.t < kSub ? lds64[g.t] : 0;
         if (own) sum_up(row.sub[stage][g.t], own);
-        if (!meet(&meets[1], S, g, s)) return false;
+        if (!meet(&meets[1], S, a.meet_ticks, g, s)) return false;
         h = g.t < kSub ? get(row.sub[stage][g.t]) : 0ull;
         double sub_below, sub_total;
         const int bf = crossing(h, T - below, sub_below, sub_total);
@@ -721,7 +720,7 @@ __device__ __forceinline__ SplitEnd split_row(const SampleArgs& a, int vec, int 
             put(me.kmax, kmax);
             put(me.kept, (uint64_t)kept);
         }
-        if (!meet(&meets[2], S, g, s)) return false;
+        if (!meet(&meets[2], S, a.meet_ticks, g, s)) return false;
         const uint32_t n_l = in ? get(segs[g.lane].n) : 0u;
         const uint32_t n = wave_sum(n_l);
         kept_l = in ? (double)get(segs[g.lane].kept) : 0.0;
@@ -832,7 +831,7 @@ __device__ __forceinline__ SplitEnd split_row(const SampleArgs& a, int vec, int 
         }
         ls = g.dsum(ls);
         if (g.t == 0) put(me.kept, (uint64_t)ls);
-        if (!meet(&row.meet[7], S, g, s)) return kEndUnsampled;
+        if (!meet(&row.meet[7], S, a.meet_ticks, g, s)) return kEndUnsampled;
         kept_l = in ? (double)get(segs[g.lane].kept) : 0.0;
     }
 
