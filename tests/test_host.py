@@ -6,6 +6,7 @@ import os
 import re
 import subprocess
 import textwrap
+import timeit
 
 import numpy as np
 import pytest
@@ -33,6 +34,27 @@ def test_library_loads_and_reports_version():
         assert hasattr(lib, s)
     lib.vxs_version.restype = __import__("ctypes").c_char_p
     assert b"gfx950" in lib.vxs_version()
+
+
+def test_array_addresses(tmp_path):
+    """ptr() of every kind of array is numpy's own address, and none takes longer than asking numpy for it."""
+    class Sub(np.ndarray):
+        pass
+
+    a = np.arange(24, dtype=np.float32).reshape(4, 6)
+    read_only = a.copy()
+    read_only.flags.writeable = False
+    arrays = [a, read_only, a[1:], a[:, ::2], a.T, np.asfortranarray(a), a.view(Sub), np.empty(0, np.int32), np.array(3.0),
+              np.broadcast_to(np.float32(1), (3, 4)), np.frombuffer(b"\0" * 32, np.int32), np.zeros(3, _lib.PARAMS_DTYPE)[1:],
+              np.memmap(tmp_path / "m", np.float32, "w+", shape=(8,))]
+    for x in arrays:
+        assert _lib.ptr(x) == x.ctypes.data
+
+    def us(fn):
+        return min(timeit.repeat(fn, number=2000, repeat=30)) / 2000 * 1e6
+
+    for x in (a, read_only, arrays[3]):
+        assert us(lambda: _lib.ptr(x)) < 1.1 * us(lambda: x.ctypes.data)
 
 
 def test_params_struct_layout(tmp_path):

@@ -160,15 +160,20 @@ def load_synth() -> ctypes.CDLL:
     return _synth
 
 
+# numpy's C struct of an array (PyArrayObject): the object header, then the address of its data.
+_DATA_AT = object.__basicsize__
+_probe = np.zeros(2)
+assert c_void_p.from_address(id(_probe) + _DATA_AT).value == _probe.ctypes.data
+
+
 def ptr(a) -> int | None:
     """Address of a numpy array / torch tensor / None (for ctypes void* arguments)."""
     if a is None:
         return None
     if isinstance(a, np.ndarray):
-        try:  # through the buffer protocol: 0.3 us where ndarray.ctypes takes 1.0 us
-            return ctypes.addressof(ctypes.c_char.from_buffer(a))
-        except (TypeError, ValueError, BufferError):  # read-only, empty or not C-contiguous
-            return a.ctypes.data
+        # 0.3 us whatever the array; ndarray.ctypes takes 1.25, the buffer protocol 0.45 and, where it
+        # refuses (read-only, empty or not C-contiguous), 1.75 with ndarray.ctypes after it
+        return c_void_p.from_address(id(a) + _DATA_AT).value
     if hasattr(a, "data_ptr"):
         return a.data_ptr()
     if isinstance(a, int):
