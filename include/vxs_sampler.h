@@ -131,7 +131,7 @@ VXS_API int vxs_sample(vxs_ctx* ctx, int rows, int vocab, const float* logits, i
  * memory (params included). Per-row errors land in out_ids as negative codes; call
  * vxs_synchronize to wait. For callers whose logits are already resident on the GPU (logit
  * heads on device) and for kernel-only timing. Batches of at most 192 rows with vocab > 8192 split
- * each row over several workgroups, in a workspace of about 29 MB that the context allocates at the
+ * each row over several workgroups, in a workspace of about 20 MB that the context allocates at the
  * first such call on a stream (its own, and up to four set with vxs_set_stream); where none is to be
  * had, and on a stream that is being captured, the call takes one workgroup per row. Same ids.
  */

@@ -2,6 +2,7 @@
 reference's options and RNG, and the product/oracle separation. No GPU calls."""
 from __future__ import annotations
 
+import ctypes
 import os
 import re
 import subprocess
@@ -89,6 +90,13 @@ def test_split_workspaces_over_streams(tmp_path):
                     os.path.join(REPO, "tests", "split_workspace.cpp"), "-o", str(exe)], check=True)
     p = subprocess.run([str(exe)], capture_output=True, text=True, timeout=60)
     assert p.returncode == 0, p.stdout
+
+
+def test_split_workspace_size():
+    """A stream's workspace for split wide rows is no larger than its 192 rows and 2048 segments need."""
+    size = _lib.load_vxs()._ZN3vxs21split_workspace_bytesEv
+    size.restype = ctypes.c_size_t
+    assert size() <= 192 * 4736 + 2048 * 9264
 
 
 def test_hip_build_flags():

@@ -281,6 +281,7 @@ std::mutex& noalloc_lock(int device);
 // which wide rows of small batches are split with (split_wanted).
 hipError_t launch_sample(const SampleArgs& a, hipStream_t stream, void* split_ws = nullptr);
 hipError_t launch_sample_wide(const SampleArgs& a, hipStream_t stream, void* split_ws);
+constexpr int kSplitMaxRows = 192;      // of one launch
 constexpr int kSplitMaxRecords = 2048;  // rows x segments of one launch
 size_t split_workspace_bytes();
 bool split_wanted(const SampleArgs& a);

@@ -1469,7 +1469,7 @@ __global__ __launch_bounds__(kTW) __attribute__((amdgpu_waves_per_eu(4))) void s
 
 }  // namespace
 
-size_t split_workspace_bytes() { return (sizeof(SplitRow) + sizeof(SplitSeg)) * (size_t)kSplitMaxRecords; }
+size_t split_workspace_bytes() { return sizeof(SplitRow) * (size_t)kSplitMaxRows + sizeof(SplitSeg) * (size_t)kSplitMaxRecords; }
 
 // Rows over several workgroups (vxs_split.h): the sweeps of 1024 entries per segment, 0 when the call is not
 // for it. Segments of 4096 entries while the call then has at most 1024 of them (four workgroups per
@@ -1487,7 +1487,7 @@ size_t split_workspace_bytes() { return (sizeof(SplitRow) + sizeof(SplitSeg)) * 
 // (300 x 20000: top-k 50 31.8 / 29.9, nucleus 40.7 / 220). On a caller's stream the workspace's event adds
 // 1.0 to 1.3 us (64 x 9001 greedy 6.7).
 static int split_segment(const SampleArgs& a) {
-    if (a.rows > 192 || a.out_logits || a.out_probs || (a.kflags & KF_STOP_AFTER_PENALTY)) return 0;
+    if (a.rows > kSplitMaxRows || a.out_logits || a.out_probs || (a.kflags & KF_STOP_AFTER_PENALTY)) return 0;
     for (int nc : {4, 10}) {
         const int len = 1024 * nc, S = (a.vocab + len - 1) / len;
         if (S <= kSplitMaxSegs && (int64_t)a.rows * S <= (nc == 4 ? 1024 : kSplitMaxRecords)) return nc;
@@ -1506,7 +1506,7 @@ hipError_t launch_sample_wide(const SampleArgs& a, hipStream_t stream, void* spl
     if (nc) {
         const int S = (a.vocab + 1024 * nc - 1) / (1024 * nc);
         SplitRow* rows = static_cast<SplitRow*>(split_ws);
-        SplitSeg* segs = reinterpret_cast<SplitSeg*>(rows + kSplitMaxRecords);
+        SplitSeg* segs = reinterpret_cast<SplitSeg*>(rows + kSplitMaxRows);
         dyn = dyn < 128u * nc ? 128u * nc : dyn;  // a segment's bitmap may be longer than a short row's
         if (nc == 4)
             hipLaunchKernelGGL(sample_split_kernel<4>, dim3(a.rows * S), dim3(kTW), dyn, stream, a, vec, S, rows, segs);
