@@ -174,6 +174,23 @@ void record_error(vxs_ctx* ctx) {
     for (int s = 2; s < 8; s++) expect(sample_on(ctx, s) == VXS_OK, "a call's status");
 }
 
+// No memory for a workspace: the calls take one workgroup per row, and few of them try to allocate.
+void no_memory(vxs_ctx* ctx) {
+    sample_on(ctx, 1);  // (the other buffers of a call are there)
+    const int before = allocations;
+    mallocs_fail = 1 << 30;
+    for (int i = 0; i < 200; i++) {
+        expect(sample_on(ctx, i % 2 ? 0 : 2) == VXS_OK, "a call's status");
+        expect(launched_with == nullptr, "no workspace");
+    }
+    expect(allocations - before <= 2, "one try, or two, in 200 calls");
+    sample_on(ctx, 1);
+    expect(launched_with != nullptr, "a stream's own workspace");
+    mallocs_fail = 0;
+    for (int i = 0; i < 300; i++) sample_on(ctx, 0);
+    expect(launched_with != nullptr, "a workspace once there is memory again");
+}
+
 void run(const char* name, void (*test)(vxs_ctx*)) {
     std::printf("%s\n", name);
     vxs_ctx* ctx = nullptr;
@@ -192,6 +209,7 @@ int main() {
     run("streams in turn", streams_in_turn);
     run("an older error", older_error);
     run("an event that cannot be recorded", record_error);
+    run("no memory", no_memory);
     std::printf("%d launches, %d failures\n", launches, failures);
     return failures != 0;
 }

@@ -83,6 +83,7 @@ struct SplitWs {
     bool recorded = false;
 };
 constexpr int kSplitStreams = 4;  // caller-supplied streams a context holds a workspace for
+constexpr int kSplitRetry = 256;  // calls without a workspace after one could not be allocated
 
 }  // namespace
 
@@ -105,6 +106,7 @@ struct vxs_ctx {
     void* noalloc = nullptr;  // this device's fixed scratch (vxs_sample_noalloc), looked up at create
     SplitWs split_own;                  // for own_stream, which outlives every use
     SplitWs split_ext[kSplitStreams];  // for streams set by the caller
+    int split_retry = 0;               // calls left before the next try to allocate one
     uint32_t meet_ticks = vxs::kMeetTicks;
 };
 
@@ -312,8 +314,12 @@ void set_resident(vxs::SampleArgs& a, const vxs_history* h, const int32_t* d_slo
     if (rng_stream >= 0) a.kflags |= vxs::KF_RNG | (rng_stream == 1 ? vxs::KF_RNG_SUB : 0u);
 }
 
-bool split_alloc(SplitWs& w, hipStream_t stream) {
+bool split_alloc(vxs_ctx* ctx, SplitWs& w, hipStream_t stream) {
     if (w.p) return true;
+    if (ctx->split_retry > 0) {
+        ctx->split_retry--;
+        return false;
+    }
     // another thread may be capturing a graph: allocating is no part of that
     hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
     (void)hipThreadExchangeStreamCaptureMode(&mode);
@@ -325,7 +331,10 @@ bool split_alloc(SplitWs& w, hipStream_t stream) {
         ok = false;
     }
     (void)hipThreadExchangeStreamCaptureMode(&mode);
-    if (!ok) (void)hipGetLastError();
+    if (!ok) {
+        (void)hipGetLastError();
+        ctx->split_retry = kSplitRetry;
+    }
     return ok;
 }
 
@@ -344,7 +353,7 @@ SplitWs* split_workspace(vxs_ctx* ctx, const vxs::SampleArgs& a) {
         return nullptr;
     }
     if (cap != hipStreamCaptureStatusNone) return nullptr;
-    if (st == ctx->own_stream) return split_alloc(ctx->split_own, st) ? &ctx->split_own : nullptr;
+    if (st == ctx->own_stream) return split_alloc(ctx, ctx->split_own, st) ? &ctx->split_own : nullptr;
     auto idle = [](SplitWs& w) { return !w.recorded || hipEventQuery(w.last) == hipSuccess; };
     SplitWs* w = nullptr;
     for (SplitWs& x : ctx->split_ext)
@@ -362,7 +371,7 @@ SplitWs* split_workspace(vxs_ctx* ctx, const vxs::SampleArgs& a) {
         w->last = nullptr;
         return nullptr;
     }
-    if (!split_alloc(*w, st)) return nullptr;
+    if (!split_alloc(ctx, *w, st)) return nullptr;
     w->stream = st;
     return w;
 }
