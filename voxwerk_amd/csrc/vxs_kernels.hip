@@ -1455,8 +1455,10 @@ template <int NC>
 hipError_t launch_nc(const SampleArgs& a, int vec, hipStream_t stream) {
     // The uniform read ahead for rows that draw from a resident store's generator and for polled host
     // calls (24-sequence device step 207 -> 195 us, frame of 15 host calls 343 -> 334); for uniforms in
-    // device memory it costs more than the one late read (256 x 3072: 11.46 us, 11.26 without).
-    // Vocabularies above 3072 are neither talker's nor code predictor's and have the one instance.
+    // device memory it costs more than the one late read (256 x 3072: 11.46 us, 11.26 without). Above 3072
+    // entries it gives and takes (us, without / with: stores 256 x 4096 nucleus 13.9 / 13.5, 16 x 5000 30.9 /
+    // 31.3, 16 x 8192 top-k 13.0 / 13.3, nucleus 24.3 / 24.0; polled 16 x 6144 27.1 / 28.0, 16 x 8192 31.6 / 33.2):
+    // one instance there.
     if constexpr (NC <= 3) {
         if ((a.kflags & KF_RNG) || a.done_flag) {
             hipLaunchKernelGGL((sample_rows_kernel<NC, true>), dim3(a.rows), dim3(kT), 0, stream, a, vec);

@@ -1473,7 +1473,8 @@ size_t split_workspace_bytes() { return sizeof(SplitRow) * (size_t)kSplitMaxRows
 
 // Rows over several workgroups (vxs_split.h): the sweeps of 1024 entries per segment, 0 when the call is not
 // for it. Segments of 4096 entries while the call then has at most 1024 of them (four workgroups per
-// compute unit), else of 10240; one workgroup per row when the call writes back, or has rows enough to keep
+// compute unit up to 155000 entries; a workgroup has room for the whole row's history bitmap, with which
+// three fit at 262144 and one at 524288), else of 10240; one workgroup per row when the call writes back, or has rows enough to keep
 // the compute units busy that way. The options are in device memory, so one limit serves them all, at the
 // rows where top-k up to about 150 still gains (us, split / one workgroup per row; nucleus top-p 0.9):
 //                 top-k 50       100         200         240         256         nucleus     greedy
