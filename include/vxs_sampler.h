@@ -98,7 +98,8 @@ VXS_API void* vxs_get_stream(const vxs_ctx* ctx);
 /*
  * The longest time, in units of 10 ns, that the workgroups of a row split over several of them
  * (vxs_sample_device) wait for each other before one samples it alone; 50000 (500 us) in a new
- * context. The ids are the same. 0 gives every such wait up, for tests of that path.
+ * context, at most 10000000 (100 ms). The ids are the same. 0 gives every such wait up, for tests of that
+ * path.
  */
 VXS_API int vxs_set_split_wait(vxs_ctx* ctx, uint32_t ticks);
 

@@ -174,6 +174,12 @@ void record_error(vxs_ctx* ctx) {
     for (int s = 2; s < 8; s++) expect(sample_on(ctx, s) == VXS_OK, "a call's status");
 }
 
+void split_wait(vxs_ctx* ctx) {
+    expect(vxs_set_split_wait(nullptr, 1) == VXS_ERR_INVALID_ARG, "no context");
+    expect(vxs_set_split_wait(ctx, 10000000) == VXS_OK, "the longest wait");
+    expect(vxs_set_split_wait(ctx, 10000001) == VXS_ERR_INVALID_ARG, "a wait too long");
+}
+
 // No memory for a workspace: the calls take one workgroup per row, and few of them try to allocate.
 void no_memory(vxs_ctx* ctx) {
     sample_on(ctx, 1);  // (the other buffers of a call are there)
@@ -210,6 +216,7 @@ int main() {
     run("an older error", older_error);
     run("an event that cannot be recorded", record_error);
     run("no memory", no_memory);
+    run("the wait of split rows", split_wait);
     std::printf("%d launches, %d failures\n", launches, failures);
     return failures != 0;
 }

@@ -671,6 +671,7 @@ VXS_API int vxs_set_stream(vxs_ctx* ctx, void* hip_stream) {
 
 VXS_API int vxs_set_split_wait(vxs_ctx* ctx, uint32_t ticks) {
     if (!ctx) return VXS_ERR_INVALID_ARG;
+    if (ticks > vxs::kMeetTicksMax) return fail(ctx, VXS_ERR_INVALID_ARG, "ticks above 100 ms");
     ctx->meet_ticks = ticks;
     return VXS_OK;
 }

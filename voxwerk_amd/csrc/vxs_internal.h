@@ -71,7 +71,8 @@ struct SampleArgs {
     vxs_params direct_params;
     uint32_t meet_ticks;  // split wide rows: the longest wait of a row's workgroups for each other (10 ns each)
 };
-constexpr uint32_t kMeetTicks = 50000;  // its default, 500 us
+constexpr uint32_t kMeetTicks = 50000;        // its default, 500 us
+constexpr uint32_t kMeetTicksMax = 10000000;  // 100 ms: a row meets up to eight times
 
 enum : int {
     kPathBlock = 0,  // one 256-thread workgroup per row
